@@ -150,6 +150,16 @@ SIGNATURES = {
         _c_vp, _c_vp, _c_vp,                    # row_tok, row_conf, counts
         _c_int, _c_int, _c_int, _c_vp,          # batch, positions, dtype, stream
     ]),
+    "fdllm_unmask_workspace_size": (_c_int, [_c_int, _c_int, _c_int, ctypes.POINTER(_c_sz)]),
+    "fdllm_unmask_step_ws": (_c_int, [
+        _c_vp, _c_i64, _c_i64, _c_int,          # as fdllm_unmask_step, up to dtype
+        _c_int, _c_int,
+        _c_vp, _c_i64,
+        _c_vp, _c_i64, _c_float, _c_i64,
+        _c_vp, _c_vp, _c_vp,
+        _c_int, _c_int, _c_int,
+        _c_vp, _c_sz, _c_vp,                    # workspace, bytes, stream
+    ]),
 }
 
 _lib = None

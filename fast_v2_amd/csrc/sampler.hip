@@ -3,13 +3,24 @@
 // temperature 0) and the unmask rule of generation_functions.py:784-807, on the GPU,
 // so the step leaves its decisions in device memory and the host reads four counters.
 //
-// Kernel 1 (one workgroup per sub-block position and sequence) reads one logits row
-// twice: pass 1 keeps the running maximum, its first index and the sum of
-// exp(l - max) (online, per 16-byte vector); pass 2 finds the first index whose
-// probability, rounded to the logits' type, equals the rounded maximum probability
-// (torch.argmax over the rounded softmax returns the first of equal values; only
-// logits within 2^-8 of the maximum can tie, so pass 2 computes probabilities for
-// those alone). Kernel 2 (one wave per sequence) applies the rule to the positions.
+// The greedy token is the first index whose probability, rounded to the logits' type,
+// equals the rounded maximum probability (torch.argmax over the rounded softmax returns
+// the first of equal values); only logits within 2^-7 of the maximum can tie.
+//
+// With a workspace (fdllm_unmask_step_ws) a row is cut into chunks of kChunk logits, one
+// workgroup each: unmask_chunks_kernel reads its chunk once into registers and writes
+// (max, its first index, sum of exp(l - max), whether a smaller logit could still tie);
+// unmask_finish_kernel, one workgroup per sequence, folds the chunks of each position,
+// re-reads only the chunks in which a tie is possible, and applies the unmask rule.
+// What bounds it: the one read of the logits. 16 x 8 positions of 152064 bf16 logits
+// (38.9 MB): 10.9 us (3.6 TB/s) + 5.0 us for the finish, against 50.0 us (128 workgroups, an
+// online rescale chain per thread and the second read) + 4.4 us for the form below.
+// 8192 logits per workgroup (four 16-byte loads per thread in flight, 2432 workgroups)
+// keep every compute unit at eight workgroups.
+//
+// Without one (fdllm_unmask_step): unmask_rows_kernel, one workgroup per position, reads
+// its row twice (pass 1: running maximum, its first index and the online sum; pass 2: the
+// first tie), then unmask_select_kernel, one wave per sequence, applies the rule.
 #include <math.h>
 
 #include "fdllm_common.h"
@@ -30,6 +41,8 @@ struct UnmaskArgs {
   float* row_conf;
   int32_t* counts;
   int B, L;
+  float4* parts;  // [B * L][n_chunks] partials of the chunked form
+  int n_chunks;
 };
 
 constexpr int kThreads = 512;
@@ -163,17 +176,15 @@ __global__ __launch_bounds__(kThreads) void unmask_rows_kernel(const UnmaskArgs 
   }
 }
 
-// One wave per sequence; lane i < L is position i of the sub-block.
-__global__ __launch_bounds__(64) void unmask_select_kernel(const UnmaskArgs a) {
-  const int b = blockIdx.x;
-  const int i = threadIdx.x;
+// The unmask rule of one sequence on one wave: lane i < L is position i of the sub-block,
+// c its confidence and tok its token.
+__device__ __forceinline__ void select_positions(const UnmaskArgs& a, int b, int i, float conf, int64_t tok) {
   const bool live = i < a.L;
   const bool fin = a.finished != nullptr && a.finished[b] != 0;
   int64_t* tp = a.tokens + b * a.tok_sb + i;
   const int64_t t = live ? *tp : 0;
   const bool masked = live && t == a.mask_id && !fin;
-  const float c = masked ? a.row_conf[b * a.L + i] : -INFINITY;
-  const int64_t tok = live ? a.row_tok[b * a.L + i] : 0;
+  const float c = masked ? conf : -INFINITY;
   bool unmask = c > a.threshold;
   // most confident masked position, first on ties (torch.argmax over the row)
   float cm = live ? c : -INFINITY;
@@ -205,23 +216,239 @@ __global__ __launch_bounds__(64) void unmask_select_kernel(const UnmaskArgs a) {
   }
 }
 
+// One wave per sequence.
+__global__ __launch_bounds__(64) void unmask_select_kernel(const UnmaskArgs a) {
+  const int b = blockIdx.x;
+  const int i = threadIdx.x;
+  const bool live = i < a.L;
+  select_positions(a, b, i, live ? a.row_conf[b * a.L + i] : -INFINITY, live ? a.row_tok[b * a.L + i] : 0);
+}
+
+// ---------------------------------------------------------------------------
+// Chunked form.
+constexpr int kChunkThreads = 256;
+constexpr int kChunkVecs = 4;  // 16-byte vectors per thread, all in flight at once
+constexpr int kChunk = kChunkThreads * kChunkVecs * 8;  // logits per workgroup
+constexpr int kFinishThreads = 512;
+
+// Row r's logits as 16-byte vectors from the aligned address at or below its start: the
+// first `mis` elements of vector 0 belong to whatever precedes the row, and vector nv - 1
+// may run past its end. Every vector holds at least one logit of the row, so an aligned
+// 16-byte load of it touches no page that the row does not.
+struct RowVecs {
+  const u32x4* v;
+  int mis, nv;
+};
+__device__ __forceinline__ RowVecs row_vecs(const UnmaskArgs& a, int b, int i) {
+  const int r = max(a.row_offset + i - a.shift, 0);
+  const uint16_t* row = a.logits + b * a.lg_sb + static_cast<int64_t>(r) * a.lg_sr;
+  const int mis = static_cast<int>((reinterpret_cast<uintptr_t>(row) & 15u) >> 1);
+  return RowVecs{reinterpret_cast<const u32x4*>(row - mis), mis, (a.V + mis + 7) / 8};
+}
+// logits 8 v - mis + 0..7 of a row, -inf where there is none
+template <typename T>
+__device__ __forceinline__ void unpack_vec(const u32x4& w, int v, int mis, int V, float* x) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    x[2 * j] = Elt<T>::lo(w[j]);
+    x[2 * j + 1] = Elt<T>::hi(w[j]);
+  }
+  const int j0 = 8 * v - mis;
+  if (j0 < 0 || j0 + 8 > V) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (j0 + j < 0 || j0 + j >= V) x[j] = -INFINITY;
+  }
+}
+
+// Whether T has a value in [m - 2^-7, m): the spacing below m is at most 2^-7 up to these
+// magnitudes (bf16: 8 significant bits, fp16: 11), larger above.
+template <typename T>
+__device__ __forceinline__ bool can_tie_below(float m);
+template <>
+__device__ __forceinline__ bool can_tie_below<bf16_t>(float m) { return m <= 2.f && m > -2.f; }
+template <>
+__device__ __forceinline__ bool can_tie_below<f16_t>(float m) { return m <= 16.f && m > -16.f; }
+
+template <typename T>
+__global__ __launch_bounds__(kChunkThreads) void unmask_chunks_kernel(const UnmaskArgs a) {
+  constexpr int NW = kChunkThreads / 64;
+  __shared__ float sm[NW], ss[NW];
+  __shared__ int si[NW], sn[NW];
+  const int chunk = blockIdx.x, i = blockIdx.y, b = blockIdx.z;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  if (chunk == 0 && i == 0 && b == 0 && tid < 4) a.counts[tid] = 0;  // the finish kernel accumulates into these
+  const RowVecs rv = row_vecs(a, b, i);
+  const int v0 = chunk * (kChunk / 8) + tid;
+  u32x4 w[kChunkVecs];
+#pragma unroll
+  for (int k = 0; k < kChunkVecs; ++k) {
+    const int v = v0 + k * kChunkThreads;
+    if (v < rv.nv) w[k] = __builtin_nontemporal_load(rv.v + v);
+  }
+  float x[kChunkVecs][8];
+  float m = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < kChunkVecs; ++k) {
+    const int v = v0 + k * kChunkThreads;
+    if (v < rv.nv) {
+      unpack_vec<T>(w[k], v, rv.mis, a.V, x[k]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[k][j] = -INFINITY;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = fmaxf(m, x[k][j]);
+  }
+  m = wave_allreduce_max(m);
+  if (lane == 0) sm[wave] = m;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NW; ++u) m = fmaxf(m, sm[u]);
+  // exp relative to the chunk's maximum (0 for a chunk of -inf: its sum is then zero; a NaN
+  // or +inf logit makes it NaN, as in a softmax)
+  const float ref = m == -INFINITY ? 0.f : m;
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < kChunkVecs; ++k)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += __builtin_amdgcn_exp2f((x[k][j] - ref) * 1.4426950408889634f);
+  int idx = 0x7fffffff;
+#pragma unroll
+  for (int k = kChunkVecs - 1; k >= 0; --k)
+#pragma unroll
+    for (int j = 7; j >= 0; --j)
+      if (x[k][j] == m) idx = 8 * (v0 + k * kChunkThreads) + j - rv.mis;
+  int near = 0;
+  if (can_tie_below<T>(m)) {  // uniform over the workgroup
+#pragma unroll
+    for (int k = 0; k < kChunkVecs; ++k)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) near |= x[k][j] < m && x[k][j] >= m - 0.0078125f;
+  }
+  s = wave_allreduce_sum(s);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) idx = min(idx, __shfl_xor(idx, o, kWave));
+  const bool any_near = __builtin_amdgcn_ballot_w64(near != 0) != 0;
+  if (lane == 0) {
+    ss[wave] = s;
+    si[wave] = idx;
+    sn[wave] = any_near;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int u = 1; u < NW; ++u) {
+      s += ss[u];
+      idx = min(idx, si[u]);
+    }
+    int nr = 0;
+    for (int u = 0; u < NW; ++u) nr |= sn[u];
+    // a chunk of -inf has no index of its own: only a row of -inf would use it
+    a.parts[(static_cast<int64_t>(b) * a.L + i) * a.n_chunks + chunk] =
+        make_float4(m, s, __int_as_float(m == -INFINITY ? 0x7fffffff : idx), __int_as_float(nr));
+  }
+}
+
+// One workgroup per sequence; wave w folds positions w, w + 8, ...
+template <typename T>
+__global__ __launch_bounds__(kFinishThreads) void unmask_finish_kernel(const UnmaskArgs a) {
+  __shared__ float s_conf[64];
+  __shared__ int s_tok[64];
+  const int b = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  for (int i = threadIdx.x >> 6; i < a.L; i += kFinishThreads / 64) {
+    const float4* parts = a.parts + (static_cast<int64_t>(b) * a.L + i) * a.n_chunks;
+    float m = -INFINITY;
+    for (int c = lane; c < a.n_chunks; c += 64) m = fmaxf(m, parts[c].x);
+    m = wave_allreduce_max(m);
+    float s = 0.f;
+    for (int c = lane; c < a.n_chunks; c += 64) {
+      const float4 p = parts[c];
+      // a NaN sum is kept; a chunk of -inf adds its zero
+      s += p.x == -INFINITY ? p.y : p.y * expf(p.x - m);
+    }
+    s = wave_allreduce_sum(s);
+    if (m == -INFINITY) s = __builtin_nanf("");  // no finite logit: no probability
+    const float pmax = rnd16<T>(1.f / s);
+    const float lo_cut = m - 0.0078125f;
+    int cand = 0x7fffffff;   // first index of the maximum (kept where no comparison holds: NaN)
+    int first = 0x7fffffff;  // first index that ties
+    for (int c0 = 0; c0 < a.n_chunks; c0 += 64) {
+      const int c = c0 + lane;
+      const float4 p = c < a.n_chunks ? parts[c] : make_float4(-INFINITY, 0.f, 0.f, 0.f);
+      const int idx = c < a.n_chunks ? __float_as_int(p.z) : 0x7fffffff;
+      if (c < a.n_chunks && p.x == m) cand = min(cand, idx);
+      const bool cut = p.x >= lo_cut;
+      if (cut && rnd16<T>(expf(p.x - m) / s) == pmax) first = min(first, idx);
+      // chunks that hold other logits close to their maximum are read again
+      uint64_t todo = __builtin_amdgcn_ballot_w64(cut && __float_as_int(p.w) != 0);
+      if (todo != 0) {
+        const RowVecs rv = row_vecs(a, b, i);
+        while (todo != 0) {
+          const int cc = c0 + __builtin_ctzll(todo);
+          todo &= todo - 1;
+          const int ve = min((cc + 1) * (kChunk / 8), rv.nv);
+          for (int v = cc * (kChunk / 8) + lane; v < ve; v += 64) {
+            float x[8];
+            unpack_vec<T>(rv.v[v], v, rv.mis, a.V, x);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const int at = 8 * v + j - rv.mis;
+              if (x[j] >= lo_cut && at < first && rnd16<T>(expf(x[j] - m) / s) == pmax) first = at;
+            }
+          }
+        }
+      }
+    }
+    cand = min(cand, first);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) cand = min(cand, __shfl_xor(cand, o, kWave));
+    if (lane == 0) {
+      s_conf[i] = pmax;
+      s_tok[i] = cand;
+      a.row_tok[b * a.L + i] = cand;
+      a.row_conf[b * a.L + i] = pmax;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const bool live = lane < a.L;
+    select_positions(a, b, lane, live ? s_conf[lane] : -INFINITY, live ? s_tok[lane] : 0);
+  }
+}
+
+// Chunks of a row, one more where a row start off a 16-byte boundary can need it.
+inline int64_t unmask_chunks(int vocab) { return (static_cast<int64_t>(vocab) + 7 + kChunk - 1) / kChunk; }
+
 }  // namespace
 }  // namespace fdllm
 
-extern "C" int fdllm_unmask_step(const void* logits, int64_t logits_stride_b, int64_t logits_stride_row,
-                                 int vocab, int row_offset, int shift, int64_t* tokens, int64_t tokens_stride_b,
-                                 uint8_t* finished, int64_t mask_id, float threshold, int64_t stop_token,
-                                 int64_t* row_tok, float* row_conf, int32_t* counts, int batch, int num_positions,
-                                 int dtype, void* stream) {
+extern "C" int fdllm_unmask_workspace_size(int vocab, int batch, int num_positions, size_t* bytes) {
   using namespace fdllm;
+  FDLLM_CHECK_ARG(bytes != nullptr && vocab > 0 && batch >= 0 && num_positions >= 0 && num_positions <= 64,
+                  "fdllm_unmask_workspace_size: need 0 <= num_positions <= 64 and vocab > 0");
+  *bytes = static_cast<size_t>(unmask_chunks(vocab)) * batch * num_positions * sizeof(float4);
+  return FDLLM_OK;
+}
+
+namespace fdllm {
+namespace {
+
+int unmask_launch(const char* what, const void* logits, int64_t logits_stride_b, int64_t logits_stride_row, int vocab,
+                  int row_offset, int shift, int64_t* tokens, int64_t tokens_stride_b, uint8_t* finished,
+                  int64_t mask_id, float threshold, int64_t stop_token, int64_t* row_tok, float* row_conf,
+                  int32_t* counts, int batch, int num_positions, int dtype, bool chunked, void* workspace,
+                  size_t workspace_bytes, void* stream) {
   FDLLM_CHECK_ARG(dtype == FDLLM_DTYPE_BF16 || dtype == FDLLM_DTYPE_F16,
-                  "fdllm_unmask_step: dtype %d unsupported (bf16 or fp16 logits)", dtype);
+                  "%s: dtype %d unsupported (bf16 or fp16 logits)", what, dtype);
   FDLLM_CHECK_ARG(batch >= 0 && num_positions >= 0 && num_positions <= 64 && vocab > 0,
-                  "fdllm_unmask_step: need 0 <= num_positions <= 64 and vocab > 0");
-  FDLLM_CHECK_ARG(shift == 0 || shift == 1, "fdllm_unmask_step: shift must be 0 or 1");
+                  "%s: need 0 <= num_positions <= 64 and vocab > 0", what);
+  FDLLM_CHECK_ARG(shift == 0 || shift == 1, "%s: shift must be 0 or 1", what);
   if (batch == 0 || num_positions == 0) return FDLLM_OK;
-  FDLLM_CHECK_ARG(batch < 65536, "fdllm_unmask_step: batch too large");
-  FDLLM_CHECK_ARG(logits && tokens && row_tok && row_conf && counts, "fdllm_unmask_step: null pointer");
+  FDLLM_CHECK_ARG(batch < 65536, "%s: batch too large", what);
+  FDLLM_CHECK_ARG(logits && tokens && row_tok && row_conf && counts, "%s: null pointer", what);
   UnmaskArgs a;
   a.logits = static_cast<const uint16_t*>(logits);
   a.lg_sb = logits_stride_b;
@@ -241,9 +468,53 @@ extern "C" int fdllm_unmask_step(const void* logits, int64_t logits_stride_b, in
   a.B = batch;
   a.L = num_positions;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  a.parts = nullptr;
+  a.n_chunks = 0;
+  if (chunked) {
+    const int64_t chunks = unmask_chunks(vocab);
+    const size_t need = static_cast<size_t>(chunks) * batch * num_positions * sizeof(float4);
+    if (workspace == nullptr || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) {
+      set_last_error("%s: workspace of %zu bytes required (got %zu)", what, need, workspace_bytes);
+      return FDLLM_ERR_WORKSPACE;
+    }
+    a.parts = static_cast<float4*>(workspace);
+    a.n_chunks = static_cast<int>(chunks);
+    const dim3 g(static_cast<unsigned>(chunks), num_positions, batch);
+    if (dtype == FDLLM_DTYPE_BF16) {
+      unmask_chunks_kernel<bf16_t><<<g, dim3(kChunkThreads), 0, s>>>(a);
+      unmask_finish_kernel<bf16_t><<<dim3(batch), dim3(kFinishThreads), 0, s>>>(a);
+    } else {
+      unmask_chunks_kernel<f16_t><<<g, dim3(kChunkThreads), 0, s>>>(a);
+      unmask_finish_kernel<f16_t><<<dim3(batch), dim3(kFinishThreads), 0, s>>>(a);
+    }
+    FDLLM_RETURN_LAUNCH_STATUS(what);
+  }
   const dim3 g1(num_positions, batch);
   if (dtype == FDLLM_DTYPE_BF16) unmask_rows_kernel<bf16_t><<<g1, dim3(kThreads), 0, s>>>(a);
   else unmask_rows_kernel<f16_t><<<g1, dim3(kThreads), 0, s>>>(a);
   unmask_select_kernel<<<dim3(batch), dim3(64), 0, s>>>(a);
-  FDLLM_RETURN_LAUNCH_STATUS("fdllm_unmask_step");
+  FDLLM_RETURN_LAUNCH_STATUS(what);
+}
+
+}  // namespace
+}  // namespace fdllm
+
+extern "C" int fdllm_unmask_step(const void* logits, int64_t logits_stride_b, int64_t logits_stride_row,
+                                 int vocab, int row_offset, int shift, int64_t* tokens, int64_t tokens_stride_b,
+                                 uint8_t* finished, int64_t mask_id, float threshold, int64_t stop_token,
+                                 int64_t* row_tok, float* row_conf, int32_t* counts, int batch, int num_positions,
+                                 int dtype, void* stream) {
+  return fdllm::unmask_launch("fdllm_unmask_step", logits, logits_stride_b, logits_stride_row, vocab, row_offset, shift,
+                              tokens, tokens_stride_b, finished, mask_id, threshold, stop_token, row_tok, row_conf,
+                              counts, batch, num_positions, dtype, false, nullptr, 0, stream);
+}
+
+extern "C" int fdllm_unmask_step_ws(const void* logits, int64_t logits_stride_b, int64_t logits_stride_row,
+                                    int vocab, int row_offset, int shift, int64_t* tokens, int64_t tokens_stride_b,
+                                    uint8_t* finished, int64_t mask_id, float threshold, int64_t stop_token,
+                                    int64_t* row_tok, float* row_conf, int32_t* counts, int batch, int num_positions,
+                                    int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  return fdllm::unmask_launch("fdllm_unmask_step_ws", logits, logits_stride_b, logits_stride_row, vocab, row_offset,
+                              shift, tokens, tokens_stride_b, finished, mask_id, threshold, stop_token, row_tok,
+                              row_conf, counts, batch, num_positions, dtype, true, workspace, workspace_bytes, stream);
 }

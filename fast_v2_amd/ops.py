@@ -82,6 +82,7 @@ class _Workspace:
 
 
 _WORKSPACE = _Workspace()
+_COUNTER_BYTES = 64 * 1024  # arrival counters at the head of a workspace
 
 
 # ---------------------------------------------------------------------------
@@ -570,13 +571,18 @@ def unmask_step(logits: torch.Tensor, tokens: torch.Tensor, mask_id: int, thresh
         raise RuntimeError("unmask_step: finished must be a contiguous bool / uint8 [B]")
     if scratch is None or scratch.row_tok.shape != (B, L) or scratch.row_tok.device != dev:
         scratch = UnmaskScratch(B, L, dev)
-    rc = _ffi.lib().fdllm_unmask_step(
+    need = ctypes.c_size_t(0)
+    _ffi.check(_ffi.lib().fdllm_unmask_workspace_size(logits.shape[2], B, L, ctypes.byref(need)),
+               "fdllm_unmask_workspace_size")
+    # past the arrival counters that other calls keep at the head of the stream's scratch
+    ws = _WORKSPACE.get(_COUNTER_BYTES + need.value, dev)
+    rc = _ffi.lib().fdllm_unmask_step_ws(
         logits.data_ptr(), logits.stride(0), logits.stride(1), logits.shape[2], int(row_offset), int(shift),
         tokens.data_ptr(), tokens.stride(0), _ptr(finished), int(mask_id), float(threshold),
         -1 if stop_token is None else int(stop_token),
         scratch.row_tok.data_ptr(), scratch.row_conf.data_ptr(), scratch.counts.data_ptr(),
-        B, L, _ffi.dtype_code(logits.dtype), _ffi.stream_ptr(dev))
-    _ffi.check(rc, "fdllm_unmask_step")
+        B, L, _ffi.dtype_code(logits.dtype), ws.data_ptr() + _COUNTER_BYTES, need.value, _ffi.stream_ptr(dev))
+    _ffi.check(rc, "fdllm_unmask_step_ws")
     return scratch
 
 

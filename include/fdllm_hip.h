@@ -425,6 +425,19 @@ int fdllm_unmask_step(const void* logits, int64_t logits_stride_b, int64_t logit
                       int64_t* row_tok, float* row_conf, int32_t* counts,
                       int batch, int num_positions, int dtype, void* stream);
 
+/* fdllm_unmask_step with device scratch: each logits row is cut over several
+ * workgroups and read once. The same outputs (row_conf may differ where a sum in another
+ * order crosses a rounding boundary of the logits' type). `workspace`
+ * (fdllm_unmask_workspace_size bytes, 16-byte aligned) needs no initialisation; calls that
+ * may overlap in time need separate ones. */
+int fdllm_unmask_workspace_size(int vocab, int batch, int num_positions, size_t* bytes);
+int fdllm_unmask_step_ws(const void* logits, int64_t logits_stride_b, int64_t logits_stride_row, int vocab,
+                         int row_offset, int shift, int64_t* tokens, int64_t tokens_stride_b,
+                         uint8_t* finished, int64_t mask_id, float threshold, int64_t stop_token,
+                         int64_t* row_tok, float* row_conf, int32_t* counts,
+                         int batch, int num_positions, int dtype, void* workspace, size_t workspace_bytes,
+                         void* stream);
+
 #ifdef __cplusplus
 } /* extern "C" */
 #endif

@@ -71,3 +71,30 @@ def test_fused_sampler_generation_matches_torch_rule(gpu):
     print(f"forwards {st_a.forwards} vs {st_b.forwards}")
     assert torch.equal(a, b)
     assert st_a.step_tokens == st_b.step_tokens
+
+
+@pytest.mark.parametrize("V", [1, 7, 8185, 8192, 8193, 16384, 24570, 32001])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("scale", [0.3, 2.0])
+def test_unmask_chunk_edges(gpu, V, dtype, scale):
+    """Rows around the 8192-logit chunks, rows that start off a 16-byte boundary (odd
+    vocabularies), leading chunks of -inf and, at the small scale, maxima that smaller
+    logits tie with after rounding (the chunks that are read again). Expected: softmax in 64
+    bits, rounded to the logits' type, first index of the maximum; the fp32 sum moves a
+    probability by under 1e-6 of itself, far inside a rounding step at these draws."""
+    g = torch.Generator().manual_seed(V + int(10 * scale))
+    B, L = 3, 5
+    raw = (torch.randn(B, L, V, generator=g) * scale).to(dtype)
+    raw[1, 2, :V // 2] = float("-inf")
+    raw[2, 1, V - 1] = 1.5 if scale < 1 else 20.0
+    p = torch.softmax(raw.double(), dim=-1).to(dtype).float()
+    top = p.max(dim=-1, keepdim=True).values
+    tok = (p == top).to(torch.uint8).argmax(dim=-1)
+    x = torch.full((B, L), V + 1, dtype=torch.int64, device=gpu)
+    print(f"case unmask chunks V={V} {dtype} scale={scale}", flush=True)
+    sc = ops.unmask_step(raw.to(gpu), x, V + 1, 2.0, row_offset=0, shift=0)
+    assert torch.equal(sc.row_tok.cpu(), tok)
+    torch.testing.assert_close(sc.row_conf.cpu(), top[..., 0], atol=0, rtol=0)
+    best = top[..., 0].argmax(dim=-1)
+    assert x.cpu().gather(1, best[:, None])[:, 0].tolist() == tok.gather(1, best[:, None])[:, 0].tolist()
+    assert sc.counts.tolist()[:2] == [B, B * (L - 1)]
