@@ -142,6 +142,14 @@ SIGNATURES = {
     ]),
     "fdllm_rope_kv_write": (_c_int, [ctypes.POINTER(RopeKVDesc), _c_vp]),
     "fdllm_qkv_rope_kv_write": (_c_int, [ctypes.POINTER(QkvRopeDesc), _c_vp]),
+    "fdllm_qkv_rope_workspace_size": (_c_int, [ctypes.POINTER(QkvRopeDesc), ctypes.POINTER(_c_sz)]),
+    "fdllm_qkv_rope_kv_write_ws": (_c_int, [ctypes.POINTER(QkvRopeDesc), _c_vp, _c_sz, _c_vp]),
+    "fdllm_linear_workspace_size": (_c_int, [_c_int, _c_int, _c_int, _c_int, ctypes.POINTER(_c_sz)]),
+    "fdllm_linear": (_c_int, [
+        _c_vp, _c_i64, _c_vp, _c_vp, _c_vp,     # x, x row stride, w, w_up, bias
+        _c_vp, _c_int, _c_int, _c_int, _c_int,  # out, rows, out_features, in_features, dtype
+        _c_vp, _c_sz, _c_vp,                    # workspace, bytes, stream
+    ]),
     "fdllm_unmask_step": (_c_int, [
         _c_vp, _c_i64, _c_i64, _c_int,          # logits, batch stride, row stride, vocab
         _c_int, _c_int,                         # row_offset, shift
@@ -209,4 +217,5 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle (the raw lookup: a Stream object takes 1.2 us to make)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)

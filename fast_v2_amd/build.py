@@ -30,8 +30,9 @@ PROBES_LIB_PATH = LIB_DIR / "libfdllm_probes.so"
 HEADER = REPO_DIR / "include" / "fdllm_hip.h"
 PROBES_HEADER = REPO_DIR / "include" / "fdllm_probes.h"
 
-SOURCES = [CSRC / "gather_rmsnorm.hip", CSRC / "block_attn.hip", CSRC / "rope_kv.hip", CSRC / "sampler.hip"]
-DEPS = SOURCES + [CSRC / "fdllm_common.h", CSRC / "attn_plan.h", CSRC / "host_errors.h", HEADER]
+SOURCES = [CSRC / "gather_rmsnorm.hip", CSRC / "block_attn.hip", CSRC / "rope_kv.hip", CSRC / "sampler.hip",
+           CSRC / "linear.hip"]
+DEPS = SOURCES + [CSRC / "fdllm_common.h", CSRC / "skinny_gemm.h", CSRC / "attn_plan.h", CSRC / "host_errors.h", HEADER]
 PROBES_SOURCES = [CSRC / "probes.hip"]
 PROBES_DEPS = PROBES_SOURCES + [PROBES_HEADER]
 

@@ -7,7 +7,7 @@
 // destination. V rows are copied in 16-byte vectors. The arithmetic rounds to the
 // 16-bit type after each product and after the sum, exactly as the eager
 // expression q * cos + rotate_half(q) * sin (utils/attention_backends.py:777-788).
-#include "fdllm_common.h"
+#include "skinny_gemm.h"
 
 namespace fdllm {
 namespace {
@@ -170,6 +170,50 @@ constexpr int kQkvBM = 128;  // token rows per tile (and head_dim: columns per t
 constexpr int kQkvKT = FDLLM_QKV_KT;  // K step per LDS slot (64 or 32)
 constexpr int kQkvYS = 136;  // epilogue tile row stride (elements; 272 bytes)
 
+// One token row's 8-dimension block c of a head and its partners 64 further on, rounded
+// projections ya / yb: rotated (q, k) or as they are (v) to every destination.
+template <typename T>
+__device__ __forceinline__ void qkv_store(const fdllm_rope_kv_desc& r, int kind, int hh, int tok, int c,
+                                          const u32x4& ya, const u32x4& yb) {
+  constexpr int half = 64;
+  const int b = tok / r.seq_len;
+  const int t = tok - b * r.seq_len;
+  auto turn = [&](u32x4& w0, u32x4& w1) __attribute__((always_inline)) {
+    if (r.cos == nullptr) {  // projections alone
+      w0 = ya;
+      w1 = yb;
+      return;
+    }
+    const uint16_t* cs = static_cast<const uint16_t*>(r.cos) + b * r.cs_stride_b + t * r.cs_stride_s;
+    const uint16_t* sn = static_cast<const uint16_t*>(r.sin) + b * r.cs_stride_b + t * r.cs_stride_s;
+    rope8<T>(ya, yb, cs, sn, c, half, w0, w1);
+  };
+  if (kind == 0) {
+    u32x4 w0, w1;
+    turn(w0, w1);
+    put_pair(r.q_out, b * r.qo_stride_b + t * r.qo_stride_s + hh * r.qo_stride_h, c, half, w0, w1);
+    return;
+  }
+  const int pos1 = (r.write_start ? r.write_start[b] : 0) + r.write_offset + t;
+  const int pos2 = r.block_offset + t;
+  const bool to_cache = r.k_cache != nullptr && pos1 >= 0 && pos1 < r.cache_len;
+  const bool to_block = r.k_block != nullptr && pos2 >= 0 && pos2 < r.block_len;
+  const int64_t o_at = b * r.ko_stride_b + t * r.ko_stride_s + hh * r.ko_stride_h;
+  const int64_t c_at = b * r.c_stride_b + pos1 * r.c_stride_s + hh * r.c_stride_h;
+  const int64_t b_at = b * r.bc_stride_b + pos2 * r.bc_stride_s + hh * r.bc_stride_h;
+  if (kind == 2) {
+    if (r.v_out) put_pair(r.v_out, o_at, c, half, ya, yb);
+    if (to_cache) put_pair(r.v_cache, c_at, c, half, ya, yb);
+    if (to_block) put_pair(r.v_block, b_at, c, half, ya, yb);
+    return;
+  }
+  u32x4 w0, w1;
+  turn(w0, w1);
+  if (r.k_out) put_pair(r.k_out, o_at, c, half, w0, w1);
+  if (to_cache) put_pair(r.k_cache, c_at, c, half, w0, w1);
+  if (to_block) put_pair(r.k_block, b_at, c, half, w0, w1);
+}
+
 // BN: columns of one head per workgroup (128: the whole head; 64: two workgroups per
 // head, each with 32 columns and their RoPE partners 64 further on); NS: LDS ring slots.
 template <typename T, bool F16, int BN, int NS>
@@ -330,40 +374,74 @@ __global__ __launch_bounds__(256) void qkv_rope_kernel(const QkvArgs a) {
   lds_barrier();
 
   // ---- rotation and stores: item = (token row, 8-dimension block c in the first half)
-  const int S = r.seq_len;
   constexpr int half = kQkvBM / 2;
   constexpr int NB = BN / 16;  // 8-dimension blocks per row in each half of this workgroup
   for (int it = tid; it < kQkvBM * NB; it += 256) {
     const int rr = it / NB;
     const int c = c0 + (it % NB) * 8;
     if (rr >= rows) break;  // items are row-major: every later item is past the end too
-    const int tok = row0 + rr;
-    const int b = tok / S;
-    const int t = tok - b * S;
     const u32x4 ya = *reinterpret_cast<const u32x4*>(Y + rr * kQkvYS + c);
     const u32x4 yb = *reinterpret_cast<const u32x4*>(Y + rr * kQkvYS + half + c);
-    const int pos1 = (r.write_start ? r.write_start[b] : 0) + r.write_offset + t;
-    const int pos2 = r.block_offset + t;
-    const bool to_cache = r.k_cache != nullptr && pos1 >= 0 && pos1 < r.cache_len;
-    const bool to_block = r.k_block != nullptr && pos2 >= 0 && pos2 < r.block_len;
-    if (kind == 2) {
-      if (r.v_out) put_pair(r.v_out, b * r.ko_stride_b + t * r.ko_stride_s + hh * r.ko_stride_h, c, half, ya, yb);
-      if (to_cache) put_pair(r.v_cache, b * r.c_stride_b + pos1 * r.c_stride_s + hh * r.c_stride_h, c, half, ya, yb);
-      if (to_block) put_pair(r.v_block, b * r.bc_stride_b + pos2 * r.bc_stride_s + hh * r.bc_stride_h, c, half, ya, yb);
-      continue;
-    }
-    const uint16_t* cs = static_cast<const uint16_t*>(r.cos) + b * r.cs_stride_b + t * r.cs_stride_s;
-    const uint16_t* sn = static_cast<const uint16_t*>(r.sin) + b * r.cs_stride_b + t * r.cs_stride_s;
-    u32x4 w0, w1;
-    rope8<T>(ya, yb, cs, sn, c, half, w0, w1);
-    if (kind == 0) {
-      put_pair(r.q_out, b * r.qo_stride_b + t * r.qo_stride_s + hh * r.qo_stride_h, c, half, w0, w1);
-    } else {
-      if (r.k_out) put_pair(r.k_out, b * r.ko_stride_b + t * r.ko_stride_s + hh * r.ko_stride_h, c, half, w0, w1);
-      if (to_cache) put_pair(r.k_cache, b * r.c_stride_b + pos1 * r.c_stride_s + hh * r.c_stride_h, c, half, w0, w1);
-      if (to_block) put_pair(r.k_block, b * r.bc_stride_b + pos2 * r.bc_stride_s + hh * r.bc_stride_h, c, half, w0, w1);
-    }
+    qkv_store<T>(r, kind, hh, row0 + rr, c, ya, yb);
   }
+}
+
+// The same projections for at most 128 token rows, on the weight-streaming kernel of
+// skinny_gemm.h (weight rows cut over K as well): the tiles above leave such a call at one
+// or two workgroups per head, 72 on the 7B layout. A weight tile is BN / 2 columns of one
+// head and their RoPE partners 64 further on.
+template <typename T>
+struct QkvEpi {
+  fdllm_qkv_rope_desc d;
+
+  __device__ __forceinline__ void where(int head, int& kind, int& hh) const {
+    const int Hq = d.rope.num_q_heads, Hkv = d.rope.num_kv_heads;
+    kind = head < Hq ? 0 : (head < Hq + Hkv ? 1 : 2);
+    hh = kind == 0 ? head : (kind == 1 ? head - Hq : head - Hq - Hkv);
+  }
+  template <int BN>
+  __device__ __forceinline__ SkinnyRows rows(int tile) const {
+    constexpr int parts = 128 / BN;
+    int kind, hh;
+    where(tile / parts, kind, hh);
+    const int c0 = (tile % parts) * (BN / 2);
+    const int K = d.hidden;
+    const uint16_t* w = static_cast<const uint16_t*>(kind == 0 ? d.wq : (kind == 1 ? d.wk : d.wv)) +
+                        (static_cast<int64_t>(hh) * 128 + c0) * K;
+    return SkinnyRows{w, w + static_cast<int64_t>(64) * K, BN / 2 * K * 2, BN / 2 * K * 2};
+  }
+  template <int BN>
+  __device__ __forceinline__ void store(int tile, int m, int blk, const f32x4 v[4]) const {
+    constexpr int parts = 128 / BN;
+    int kind, hh;
+    where(tile / parts, kind, hh);
+    const int c = (tile % parts) * (BN / 2) + blk * 8;
+    const uint16_t* bias = static_cast<const uint16_t*>(kind == 0 ? d.bq : (kind == 1 ? d.bk : d.bv));
+    u32x4 y[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float f[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = v[2 * h + (j >> 2)][j & 3];
+      if (bias != nullptr) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] += Elt<T>::lo(static_cast<uint32_t>(bias[hh * 128 + 64 * h + c + j]));
+      }
+      y[h] = pack8<T>(f);
+    }
+    qkv_store<T>(d.rope, kind, hh, m, c, y[0], y[1]);
+  }
+};
+
+constexpr int kSkinnyBN = 64;
+
+SkinnyArgs skinny_qkv_plan(const fdllm_qkv_rope_desc& d, bool workspace) {
+  SkinnyArgs a = {};
+  a.T = d.rope.batch * d.rope.seq_len;
+  a.ku = d.hidden / 64;
+  a.tiles = (d.rope.num_q_heads + 2 * d.rope.num_kv_heads) * (128 / kSkinnyBN);
+  skinny_plan(a, workspace);
+  return a;
 }
 
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -406,8 +484,21 @@ extern "C" int fdllm_rope_kv_write(const fdllm_rope_kv_desc* d, void* stream) {
   FDLLM_RETURN_LAUNCH_STATUS("fdllm_rope_kv_write");
 }
 
-extern "C" int fdllm_qkv_rope_kv_write(const fdllm_qkv_rope_desc* d, void* stream) {
-  using namespace fdllm;
+namespace fdllm {
+namespace {
+
+bool qkv_empty(const fdllm_qkv_rope_desc& d) {
+  return d.rope.batch == 0 || d.rope.seq_len == 0 || d.rope.num_q_heads + d.rope.num_kv_heads == 0;
+}
+
+// 64-row weight tiles whose partial sums have counters and whose rows stay within 32 bits
+bool qkv_skinny(const fdllm_qkv_rope_desc& d) {
+  return static_cast<int64_t>(d.rope.batch) * d.rope.seq_len <= kSkinnyMaxRows &&
+         static_cast<int64_t>(d.rope.num_q_heads) + 2 * static_cast<int64_t>(d.rope.num_kv_heads) <= 65536;
+}
+
+// plain: cos / sin may be absent together where the few-row form runs
+int check_qkv(const fdllm_qkv_rope_desc* d, bool plain) {
   FDLLM_CHECK_ARG(d != nullptr, "fdllm_qkv_rope_kv_write: null descriptor");
   const fdllm_rope_kv_desc& r = d->rope;
   FDLLM_CHECK_ARG(r.dtype == FDLLM_DTYPE_BF16 || r.dtype == FDLLM_DTYPE_F16,
@@ -420,10 +511,11 @@ extern "C" int fdllm_qkv_rope_kv_write(const fdllm_qkv_rope_desc* d, void* strea
   FDLLM_CHECK_ARG(d->x_stride_row >= d->hidden && d->x_stride_row % 8 == 0 && d->x_stride_row <= (1 << 22),
                   "fdllm_qkv_rope_kv_write: x_stride_row %lld must be a multiple of 8, at least hidden",
                   static_cast<long long>(d->x_stride_row));
-  if (r.batch == 0 || r.seq_len == 0 || r.num_q_heads + r.num_kv_heads == 0) return FDLLM_OK;
+  if (qkv_empty(*d)) return FDLLM_OK;
   const int64_t T = static_cast<int64_t>(r.batch) * r.seq_len;
   FDLLM_CHECK_ARG(T < (int64_t{1} << 30), "fdllm_qkv_rope_kv_write: too many tokens");
-  FDLLM_CHECK_ARG(d->x && d->wq && d->wk && d->wv && r.cos && r.sin && r.q_out, "fdllm_qkv_rope_kv_write: null pointer");
+  FDLLM_CHECK_ARG(d->x && d->wq && d->wk && d->wv && r.q_out, "fdllm_qkv_rope_kv_write: null pointer");
+  FDLLM_CHECK_ARG(r.cos && r.sin || plain && !r.cos && !r.sin && qkv_skinny(*d), "fdllm_qkv_rope_kv_write: null cos / sin");
   FDLLM_CHECK_ARG((r.k_out == nullptr) == (r.v_out == nullptr) && (r.k_cache == nullptr) == (r.v_cache == nullptr) &&
                       (r.k_block == nullptr) == (r.v_block == nullptr),
                   "fdllm_qkv_rope_kv_write: k and v destinations must be given together");
@@ -436,6 +528,51 @@ extern "C" int fdllm_qkv_rope_kv_write(const fdllm_qkv_rope_desc* d, void* strea
                              r.c_stride_h, r.bc_stride_b, r.bc_stride_s, r.bc_stride_h};
   for (int64_t st : strides)
     FDLLM_CHECK_ARG(st % 8 == 0, "fdllm_qkv_rope_kv_write: strides must be multiples of 8 elements");
+  return FDLLM_OK;
+}
+
+}  // namespace
+}  // namespace fdllm
+
+extern "C" int fdllm_qkv_rope_workspace_size(const fdllm_qkv_rope_desc* d, size_t* bytes) {
+  using namespace fdllm;
+  FDLLM_CHECK_ARG(bytes != nullptr, "fdllm_qkv_rope_workspace_size: null pointer");
+  const int rc = check_qkv(d, true);
+  if (rc != FDLLM_OK) return rc;
+  *bytes = qkv_empty(*d) || !qkv_skinny(*d) ? 0 : skinny_workspace(skinny_qkv_plan(*d, true), kSkinnyBN);
+  return FDLLM_OK;
+}
+
+extern "C" int fdllm_qkv_rope_kv_write(const fdllm_qkv_rope_desc* d, void* stream) {
+  const int rc = fdllm::check_qkv(d, false);
+  if (rc != FDLLM_OK) return rc;
+  return fdllm_qkv_rope_kv_write_ws(d, nullptr, 0, stream);
+}
+
+extern "C" int fdllm_qkv_rope_kv_write_ws(const fdllm_qkv_rope_desc* d, void* workspace, size_t workspace_bytes,
+                                          void* stream) {
+  using namespace fdllm;
+  const int rc = check_qkv(d, true);
+  if (rc != FDLLM_OK || qkv_empty(*d)) return rc;
+  const fdllm_rope_kv_desc& r = d->rope;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int64_t T = static_cast<int64_t>(r.batch) * r.seq_len;
+  if (qkv_skinny(*d)) {
+    // 16 x 8 rows of the 7B layout: 26.5 us on the tiles below (72 workgroups), 18.1 here
+    SkinnyArgs k = skinny_qkv_plan(*d, workspace != nullptr);
+    const size_t need = skinny_workspace(k, kSkinnyBN);
+    FDLLM_CHECK_ARG(workspace == nullptr || (workspace_bytes >= need && al16(workspace)),
+                    "fdllm_qkv_rope_kv_write: workspace of %zu bytes, need %zu, 16-byte aligned", workspace_bytes, need);
+    k.x = static_cast<const uint16_t*>(d->x);
+    k.x_bytes = static_cast<int>(((T - 1) * d->x_stride_row + d->hidden) * 2);
+    k.x_stride_b = static_cast<int>(d->x_stride_row * 2);
+    k.w_stride_b = d->hidden * 2;
+    k.cnt = static_cast<int*>(workspace);
+    k.part = static_cast<uint8_t*>(workspace) + kSkinnyCounterBytes;
+    if (r.dtype == FDLLM_DTYPE_BF16) skinny_launch<false, kSkinnyBN>(k, QkvEpi<bf16_t>{*d}, s);
+    else skinny_launch<true, kSkinnyBN>(k, QkvEpi<f16_t>{*d}, s);
+    FDLLM_RETURN_LAUNCH_STATUS("fdllm_qkv_rope_kv_write");
+  }
   QkvArgs a;
   a.d = *d;
   a.T = static_cast<int>(T);
@@ -443,14 +580,13 @@ extern "C" int fdllm_qkv_rope_kv_write(const fdllm_qkv_rope_desc* d, void* strea
   const int heads = r.num_q_heads + 2 * r.num_kv_heads;
   FDLLM_CHECK_ARG(static_cast<int64_t>(a.n_mt) * heads * 2 < (int64_t{1} << 30), "fdllm_qkv_rope_kv_write: too many tiles");
   // Whole-head tiles while they give the compute units more than half a workgroup each;
-  // with fewer (the 128-row sub-block forward: 36 tiles), half-head tiles, twice as many
-  // workgroups each streaming 3/4 of the bytes: 29 against 41 us on the 7B layout (at 512
-  // rows the half-head form, 288 workgroups for 256 compute units, took 55 against 40 us).
+  // with fewer (few heads), half-head tiles, twice as many workgroups each streaming 3/4 of
+  // the bytes (36 whole-head tiles of the 7B layout: 29 against 41 us; at 512 rows the
+  // half-head form, 288 workgroups for 256 compute units, took 55 against 40 us).
   const bool half_head = a.n_mt * heads <= 128;
   a.n_tiles = a.n_mt * heads * (half_head ? 2 : 1);
   a.per_xcd = (a.n_tiles + 7) / 8;
   const dim3 grid(static_cast<unsigned>(8 * a.per_xcd));
-  hipStream_t s = static_cast<hipStream_t>(stream);
   if (r.dtype == FDLLM_DTYPE_BF16) {
     if (half_head) qkv_rope_kernel<bf16_t, false, 64, 5><<<grid, dim3(256), 0, s>>>(a);
     else qkv_rope_kernel<bf16_t, false, 128, 4><<<grid, dim3(256), 0, s>>>(a);

@@ -97,12 +97,11 @@ class RMSNorm(nn.Module):
 
 
 def set_fused_norms(model: nn.Module, on: bool) -> None:
-    """Switch every RMSNorm of ``model`` to the fused kernels, and the MLPs' SiLU-gated
-    product to its kernel (or both back to torch)."""
+    """Switch every RMSNorm of ``model`` to the fused kernels, the MLPs' SiLU-gated product
+    to its kernel, and the linear layers of calls of few rows to the weight-streaming
+    kernels (or all back to torch)."""
     for mod in model.modules():
-        if isinstance(mod, RMSNorm):
-            mod.fused = on
-        elif isinstance(mod, MLP):
+        if isinstance(mod, (RMSNorm, Attention, MLP, BlockDiffusionLM)):
             mod.fused = on
 
 
@@ -116,6 +115,7 @@ class Attention(nn.Module):
         self.k_proj = nn.Linear(cfg.hidden_size, cfg.num_key_value_heads * self.head_dim, bias=True)
         self.v_proj = nn.Linear(cfg.hidden_size, cfg.num_key_value_heads * self.head_dim, bias=True)
         self.o_proj = nn.Linear(cfg.num_attention_heads * self.head_dim, cfg.hidden_size, bias=False)
+        self.fused = False  # read by the patched forward
 
     def forward(self, *args, **kwargs):
         raise RuntimeError("attention layers run through patch_attention_layers "
@@ -132,8 +132,8 @@ class MLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.fused:
-            from .. import ops
-            return self.down_proj(ops.silu_mul(self.gate_proj(x), self.up_proj(x)))
+            from ..utils.linear_layers import gated, project
+            return project(self.down_proj, gated(self.gate_proj, self.up_proj, x))
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
 
@@ -187,6 +187,7 @@ class BlockDiffusionLM(nn.Module):
         self.config = cfg
         self.model = Backbone(cfg)
         self.lm_head = nn.Linear(cfg.hidden_size, cfg.vocab_size, bias=False)
+        self.fused = False
 
     @torch.no_grad()
     def init_weights(self, seed: int = 0) -> None:
@@ -235,6 +236,9 @@ class BlockDiffusionLM(nn.Module):
         h = self.model.norm(h) if m is None else self.model.norm.add_norm(h, m)[1]
         if logits_to_keep:
             h = h[:, -logits_to_keep:]
+        if self.fused:
+            from ..utils.linear_layers import project
+            return project(self.lm_head, h)
         return self.lm_head(h)
 
 

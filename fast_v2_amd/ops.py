@@ -23,6 +23,7 @@ in the manner of ``_wrap_flash_kvcache_as_custom_op``
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from typing import Optional, Tuple
 
@@ -70,8 +71,7 @@ class _Workspace:
         self._retired: list = []
 
     def get(self, nbytes: int, device: torch.device) -> torch.Tensor:
-        stream = torch.cuda.current_stream(device)
-        key = (device.index, stream.cuda_stream)
+        key = (device.index, _ffi.stream_ptr(device))
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < nbytes:
             if buf is not None:
@@ -480,6 +480,58 @@ def rope_kv_write(
     return (q_out, kv_o) if kv_out else q_out
 
 
+def _qkv_desc(x, wq, bq, wk, bk, wv, bv, head_dim):
+    """The projections' part of a QkvRopeDesc, (B, S, Hq, Hkv, D, device), and the tensors
+    it points to that were made here."""
+    if x.dim() != 3:
+        raise RuntimeError("qkv_rope_kv_write: x must be [B, S, hidden]")
+    B, S, H = x.shape
+    D = head_dim
+    if wq.dim() != 2 or wk.dim() != 2 or wk.shape != wv.shape or wq.shape[1] != H or wk.shape[1] != H or \
+            wq.shape[0] % D or wk.shape[0] % D:
+        raise RuntimeError("qkv_rope_kv_write: weights must be [heads * head_dim, hidden]")
+    Hq, Hkv = wq.shape[0] // D, wk.shape[0] // D
+    for name, b_, w_ in (("bq", bq, wq), ("bk", bk, wk), ("bv", bv, wv)):
+        if b_ is not None and (b_.dim() != 1 or b_.shape[0] != w_.shape[0]):
+            raise RuntimeError(f"qkv_rope_kv_write: {name} must be [{w_.shape[0]}]")
+    ts = [x, wq, wk, wv] + [b_ for b_ in (bq, bk, bv) if b_ is not None]
+    dev = _require_gpu(*ts)
+    if x.dtype not in (torch.bfloat16, torch.float16) or any(t.dtype != x.dtype for t in ts):
+        raise RuntimeError("qkv_rope_kv_write: all tensors must share one 16-bit dtype")
+    if x.stride(-1) != 1 or x.stride(1) % 8 or (B > 1 and x.stride(0) != S * x.stride(1)):
+        x = x.contiguous()
+    wq, wk, wv = (w_.contiguous() for w_ in (wq, wk, wv))
+    bq, bk, bv = (b_.contiguous() if b_ is not None else None for b_ in (bq, bk, bv))
+    d = _ffi.QkvRopeDesc()
+    d.x, d.x_stride_row, d.hidden = x.data_ptr(), x.stride(1), H
+    d.wq, d.wk, d.wv = wq.data_ptr(), wk.data_ptr(), wv.data_ptr()
+    d.bq, d.bk, d.bv = _ptr(bq), _ptr(bk), _ptr(bv)
+    return d, (B, S, Hq, Hkv, D, dev), (x, wq, wk, wv, bq, bk, bv)
+
+
+_QKV_BYTES: dict = {}  # (rows, heads, KV heads, head_dim, hidden) -> workspace bytes
+
+
+def _launch_qkv(d, dims):
+    B, S, dev = dims[0], dims[1], dims[5]
+    L = _ffi.lib()
+    ws_ptr, ws_bytes = None, 0
+    if B * S <= LINEAR_MAX_ROWS:  # the form that cuts the weights over K has partial sums
+        need = _QKV_BYTES.get((B * S, *dims[2:5], d.hidden))
+        if need is None:
+            size = ctypes.c_size_t(0)
+            _ffi.check(L.fdllm_qkv_rope_workspace_size(ctypes.byref(d), ctypes.byref(size)),
+                       "fdllm_qkv_rope_workspace_size")
+            need = size.value
+            if len(_QKV_BYTES) < 1024:
+                _QKV_BYTES[(B * S, *dims[2:5], d.hidden)] = need
+        if need:
+            ws = _WORKSPACE.get(need, dev)
+            ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+    _ffi.check(L.fdllm_qkv_rope_kv_write_ws(ctypes.byref(d), ws_ptr, ws_bytes, _ffi.stream_ptr(dev)),
+               "fdllm_qkv_rope_kv_write")
+
+
 def qkv_rope_kv_write(
     x: torch.Tensor,
     wq: torch.Tensor, bq: Optional[torch.Tensor],
@@ -503,35 +555,102 @@ def qkv_rope_kv_write(
     (utils/attention_backends.py:837-842). The projections sum in fp32 and round once
     after the bias, as a 16-bit linear layer does, in a different order than a library
     GEMM. head_dim 128, hidden a multiple of 64."""
-    if x.dim() != 3:
-        raise RuntimeError("qkv_rope_kv_write: x must be [B, S, hidden]")
-    B, S, H = x.shape
-    D = head_dim
-    if wq.dim() != 2 or wk.dim() != 2 or wk.shape != wv.shape or wq.shape[1] != H or wk.shape[1] != H or \
-            wq.shape[0] % D or wk.shape[0] % D:
-        raise RuntimeError("qkv_rope_kv_write: weights must be [heads * head_dim, hidden]")
-    Hq, Hkv = wq.shape[0] // D, wk.shape[0] // D
-    for name, b_, w_ in (("bq", bq, wq), ("bk", bk, wk), ("bv", bv, wv)):
-        if b_ is not None and (b_.dim() != 1 or b_.shape[0] != w_.shape[0]):
-            raise RuntimeError(f"qkv_rope_kv_write: {name} must be [{w_.shape[0]}]")
-    ts = [x, wq, wk, wv] + [b_ for b_ in (bq, bk, bv) if b_ is not None]
-    dev = _require_gpu(*ts)
-    if x.dtype not in (torch.bfloat16, torch.float16) or any(t.dtype != x.dtype for t in ts):
-        raise RuntimeError("qkv_rope_kv_write: all tensors must share one 16-bit dtype")
-    if x.stride(-1) != 1 or x.stride(1) % 8 or (B > 1 and x.stride(0) != S * x.stride(1)):
-        x = x.contiguous()
-    wq, wk, wv = (w_.contiguous() for w_ in (wq, wk, wv))
-    bq, bk, bv = (b_.contiguous() if b_ is not None else None for b_ in (bq, bk, bv))
-    d = _ffi.QkvRopeDesc()
-    q_out, kv_o, keep = _rope_dest_desc(d.rope, B, S, Hq, Hkv, D, x.dtype, dev, cos, sin, k_cache, v_cache,
+    d, dims, keep = _qkv_desc(x, wq, bq, wk, bk, wv, bv, head_dim)
+    B, S, Hq, Hkv, D, dev = dims
+    q_out, kv_o, kept = _rope_dest_desc(d.rope, B, S, Hq, Hkv, D, x.dtype, dev, cos, sin, k_cache, v_cache,
                                         write_start, write_offset, k_block, v_block, block_offset, q_out, kv_out)
-    d.x, d.x_stride_row, d.hidden = x.data_ptr(), x.stride(1), H
-    d.wq, d.wk, d.wv = wq.data_ptr(), wk.data_ptr(), wv.data_ptr()
-    d.bq, d.bk, d.bv = _ptr(bq), _ptr(bk), _ptr(bv)
-    rc = _ffi.lib().fdllm_qkv_rope_kv_write(ctypes.byref(d), _ffi.stream_ptr(dev))
-    del keep  # launched: the stream orders any reuse of that memory after the kernel
-    _ffi.check(rc, "fdllm_qkv_rope_kv_write")
+    _launch_qkv(d, dims)
+    del keep, kept  # launched: the stream orders any reuse of that memory after the kernel
     return (q_out, kv_o) if kv_out else q_out
+
+
+def qkv_linear(x, wq, bq, wk, bk, wv, bv, head_dim: int = 128):
+    """The projections of ``qkv_rope_kv_write`` alone, bit for bit: (q [B, S, Hq, D], k, v
+    [B, S, Hkv, D]) for at most 128 rows."""
+    d, dims, keep = _qkv_desc(x, wq, bq, wk, bk, wv, bv, head_dim)
+    B, S, Hq, Hkv, D, dev = dims
+    if B * S > LINEAR_MAX_ROWS:
+        raise RuntimeError(f"qkv_linear: {B * S} rows (at most {LINEAR_MAX_ROWS})")
+    q, k, v = (torch.empty((B, S, h, D), dtype=x.dtype, device=dev) for h in (Hq, Hkv, Hkv))
+    r = d.rope
+    r.q_out, (r.qo_stride_b, r.qo_stride_s, r.qo_stride_h) = q.data_ptr(), q.stride()[:3]
+    r.k_out, r.v_out = k.data_ptr(), v.data_ptr()
+    r.ko_stride_b, r.ko_stride_s, r.ko_stride_h = k.stride()[:3]
+    r.batch, r.seq_len, r.num_q_heads, r.num_kv_heads, r.head_dim = B, S, Hq, Hkv, D
+    r.dtype = _ffi.dtype_code(x.dtype)
+    _launch_qkv(d, dims)
+    del keep
+    return q, k, v
+
+
+LINEAR_MAX_ROWS = 128  # token rows of ``linear`` and ``gated_linear``
+
+
+def linear_fits(x: torch.Tensor, *weights: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
+    """Whether ``linear`` (``gated_linear`` with two weights) takes this layer: at most 128
+    rows of a 16-bit type, in_features a multiple of 64 (at most 65536), out_features a
+    multiple of 8, contiguous aligned weights on x's device, nothing to differentiate.
+    Below 128 rows a layer is bound by reading its weights once; above, by the products,
+    where the library's tiles are the better ones."""
+    w = weights[0]
+    if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or x.dim() < 2 or w.dim() != 2:
+        return False
+    n, k = w.shape
+    if x.shape[-1] != k or k % 64 or not 64 <= k <= 65536 or n % 8 or not 0 < n <= 1 << 24 or \
+            not 0 < x.numel() <= LINEAR_MAX_ROWS * k:
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or any(t.requires_grad for t in weights) or
+                                    (bias is not None and bias.requires_grad)):
+        return False
+    if bias is not None and (bias.dtype != x.dtype or bias.device != x.device or bias.shape != (n,) or
+                             not bias.is_contiguous() or bias.data_ptr() % 16):
+        return False
+    return all(t.dtype == x.dtype and t.device == x.device and t.shape == w.shape and t.is_contiguous() and
+               t.data_ptr() % 16 == 0 for t in weights)
+
+
+@functools.lru_cache(maxsize=1024)
+def _linear_bytes(m: int, n: int, k: int, gated: bool) -> int:
+    need = ctypes.c_size_t(0)
+    _ffi.check(_ffi.lib().fdllm_linear_workspace_size(m, n, k, gated, ctypes.byref(need)),
+               "fdllm_linear_workspace_size")
+    return need.value
+
+
+def _linear(x, w, w_up, bias):
+    k = x.shape[-1]
+    x2 = x.reshape(-1, k)
+    if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.stride(0) < k or x2.stride(0) > 1 << 22 or x2.data_ptr() % 16:
+        x2 = x2.contiguous() if not x2.is_contiguous() else x2.clone()
+    m, n = x2.shape[0], w.shape[0]
+    out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    ws_ptr, ws_bytes = None, 0
+    need = _linear_bytes(m, n, k, w_up is not None)
+    if need:
+        ws = _WORKSPACE.get(need, x.device)
+        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+    rc = _ffi.lib().fdllm_linear(x2.data_ptr(), x2.stride(0), w.data_ptr(), _ptr(w_up), _ptr(bias), out.data_ptr(), m, n, k,
+                        _ffi.dtype_code(x.dtype), ws_ptr, ws_bytes, _ffi.stream_ptr(x.device))
+    _ffi.check(rc, "fdllm_linear")
+    return out
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``x @ weight.T + bias`` of at most 128 rows (F.linear's shapes), summed in fp32 and
+    rounded once; the weights are streamed once (``linear_fits`` states what it takes)."""
+    if not linear_fits(x, weight, bias=bias):
+        raise RuntimeError(f"linear: unsupported layer (x {tuple(x.shape)} {x.dtype} on {x.device}, weight "
+                           f"{tuple(weight.shape)} {weight.dtype})")
+    return _linear(x, weight, None, bias)
+
+
+def gated_linear(x: torch.Tensor, gate_weight: torch.Tensor, up_weight: torch.Tensor) -> torch.Tensor:
+    """``silu(x @ gate_weight.T) * (x @ up_weight.T)`` of at most 128 rows in one kernel,
+    rounded where the two layers and ``silu_mul`` round (modeling.py:164)."""
+    if not linear_fits(x, gate_weight, up_weight):
+        raise RuntimeError(f"gated_linear: unsupported layers (x {tuple(x.shape)} {x.dtype} on {x.device}, weights "
+                           f"{tuple(gate_weight.shape)} {gate_weight.dtype})")
+    return _linear(x, gate_weight, up_weight, None)
 
 
 class UnmaskScratch:

@@ -31,6 +31,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import _ffi, ops
+from .linear_layers import project, streams
 from .static_kv_cache import StaticKVCache
 
 logger = logging.getLogger(__name__)
@@ -172,10 +173,11 @@ FUSED_ROPE_CACHE_WRITE = True
 # True: with the fused RoPE + cache write, the q / k / v projections run in the same
 # kernel (ops.qkv_rope_kv_write) where head_dim is 128, hidden a multiple of 64 and the
 # call has at most FUSED_QKV_MAX_TOKENS token rows. Off by default: the projections are
-# then three nn.Linear calls, as in the reference's code, and bit-identical to them; the
+# then three nn.Linear calls, as in the reference's code, and bit-identical to them, but
+# for layers marked ``fused`` in calls of at most 128 rows; the
 # fused kernel sums in another order, so its projections differ from a library GEMM's
 # in the last bit of about 1 % of the values. On the 7B layout it takes 40 us against
-# 53 us for three hipBLASLt GEMMs + the RoPE kernel at 512 rows and 29 against 53 us at
+# 53 us for three hipBLASLt GEMMs + the RoPE kernel at 512 rows and 18 against 54 us at
 # 128 rows, but 117 against 99 us at 2048 rows, where the library GEMMs' larger tiles win.
 FUSED_QKV_PROJECTION = False
 FUSED_QKV_MAX_TOKENS = 1024
@@ -234,6 +236,14 @@ def _fusable(attn_module, hidden_states, head_dim):
     return rope_ok, proj_ok
 
 
+def _streams_qkv(attn_module, hidden_states, head_dim):
+    """Whether a layer marked ``fused`` takes the kernel that streams the projections'
+    weights: calls of at most 128 rows (one kernel of 18 us at 16 x 8 rows of the 7B layout
+    against 54 for three GEMMs and the RoPE kernel)."""
+    return (getattr(attn_module, "fused", False) and head_dim == 128 and hidden_states.dim() == 3 and
+            streams(hidden_states, attn_module.q_proj, attn_module.k_proj, attn_module.v_proj))
+
+
 def _create_patched_attention_forward(attn_module, attn_backend, static_block_cache=None):
     """Attention forward over the static cache (attention_backends.py:791-898):
     q/k/v projections -> RoPE -> sub-block cache -> KV write -> block attention
@@ -254,12 +264,15 @@ def _create_patched_attention_forward(attn_module, attn_backend, static_block_ca
                                     replace_position, **kwargs)
         input_shape = hidden_states.shape[:-1]
         hidden_shape = (*input_shape, -1, head_dim)
+
+        def o_proj(x):
+            return project(attn_module.o_proj, x) if getattr(attn_module, "fused", False) else attn_module.o_proj(x)
         cos, sin = position_embeddings
         fused = attn_backend.name == AttentionBackend.HIP and FUSED_ROPE_CACHE_WRITE
         rope_ok, proj_ok = _fusable(attn_module, hidden_states, head_dim) if fused else (False, False)
-        if proj_ok and hidden_states.dim() == 3:
-            qp, kp, vp = attn_module.q_proj, attn_module.k_proj, attn_module.v_proj
-
+        qp, kp, vp = attn_module.q_proj, attn_module.k_proj, attn_module.v_proj
+        few = attn_backend.name == AttentionBackend.HIP and _streams_qkv(attn_module, hidden_states, head_dim)
+        if (proj_ok or (few and rope_ok)) and hidden_states.dim() == 3:
             def rope(kc, vc, **dst):
                 return ops.qkv_rope_kv_write(hidden_states, qp.weight, qp.bias, kp.weight, kp.bias, vp.weight,
                                              vp.bias, cos, sin, kc, vc, head_dim=head_dim, **dst)
@@ -270,10 +283,14 @@ def _create_patched_attention_forward(attn_module, attn_backend, static_block_ca
                 out = attn_backend.flash_kvcache_attention(q, full_k, full_v,
                                                            cache_seqlens=past_key_value.scratch_seqlens,
                                                            is_causal=False, scaling=scaling)
-                return attn_module.o_proj(out.reshape(*input_shape, -1))
-        q = attn_module.q_proj(hidden_states).view(hidden_shape)
-        k = attn_module.k_proj(hidden_states).view(hidden_shape)
-        v = attn_module.v_proj(hidden_states).view(hidden_shape)
+                return o_proj(out.reshape(*input_shape, -1))
+        if few:  # the same projections as above, bit for bit
+            q, k, v = ops.qkv_linear(hidden_states, qp.weight, qp.bias, kp.weight, kp.bias, vp.weight, vp.bias,
+                                     head_dim)
+        else:
+            q = qp(hidden_states).view(hidden_shape)
+            k = kp(hidden_states).view(hidden_shape)
+            v = vp(hidden_states).view(hidden_shape)
 
         if rope_ok:
             def rope(kc, vc, **dst):
@@ -285,7 +302,7 @@ def _create_patched_attention_forward(attn_module, attn_backend, static_block_ca
                 out = attn_backend.flash_kvcache_attention(q_rot, full_k, full_v,
                                                            cache_seqlens=past_key_value.scratch_seqlens,
                                                            is_causal=False, scaling=scaling)
-                return attn_module.o_proj(out.reshape(*input_shape, -1))
+                return o_proj(out.reshape(*input_shape, -1))
         q, k = _apply_rotary_pos_emb(q, k, cos, sin)
 
         if block_past_key_values is not None:
@@ -308,7 +325,7 @@ def _create_patched_attention_forward(attn_module, attn_backend, static_block_ca
         out = attn_backend.flash_kvcache_attention(q, full_k, full_v, cache_seqlens=past_key_value.scratch_seqlens,
                                                    is_causal=False, scaling=scaling)
         out = out.reshape(*input_shape, -1)
-        return attn_module.o_proj(out)
+        return o_proj(out)
 
     return patched_forward
 

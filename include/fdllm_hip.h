@@ -393,6 +393,41 @@ typedef struct fdllm_qkv_rope_desc {
 
 int fdllm_qkv_rope_kv_write(const fdllm_qkv_rope_desc* desc, void* stream);
 
+/* fdllm_qkv_rope_kv_write with device scratch, for calls of at most 128 token rows: the
+ * weight rows are cut over the K dimension as well, and the parts' fp32 sums meet in
+ * `workspace` (fdllm_qkv_rope_workspace_size bytes, 0 above 128 rows; counters in its first
+ * 64 KiB as in fdllm_linear). With cos and sin NULL (at most 128 rows) q and k are stored as
+ * projected. */
+int fdllm_qkv_rope_workspace_size(const fdllm_qkv_rope_desc* desc, size_t* bytes);
+int fdllm_qkv_rope_kv_write_ws(const fdllm_qkv_rope_desc* desc, void* workspace, size_t workspace_bytes,
+                               void* stream);
+
+/* -------------------------------------------------------------------------
+ * A linear layer of a few token rows, or the two input projections of a SiLU-gated MLP.
+ *
+ *   w_up NULL:  out[m, n] = round(x[m] . w[n] + bias[n])          (bias NULL: none)
+ *   w_up given: out[m, n] = round(round(silu(round(x[m] . w[n]))) * round(x[m] . w_up[n]))
+ *
+ * for m < rows (at most 128) and n < out_features (a multiple of 8). x has row stride
+ * x_stride_row (elements, a multiple of 8, at least in_features); w, w_up are
+ * [out_features, in_features] with contiguous rows (nn.Linear weights), in_features a
+ * multiple of 64; out is [rows, out_features], contiguous. Products are summed in fp32
+ * (MFMA) and rounded once to `dtype`; the summation order differs from a library GEMM's.
+ *
+ * `workspace` (fdllm_linear_workspace_size bytes) holds arrival counters in its first
+ * 64 KiB, which must be zero on entry and are left at zero (the layout of
+ * fdllm_kv_attn_fwd's, which may share the buffer in stream order), and fp32 partial sums.
+ * Without one (NULL) the weight rows are not cut over more workgroups than there are
+ * 64-row tiles: slower where out_features is small.
+ *
+ * Replaces: o_proj, gate_proj / up_proj / act_fn, down_proj and lm_head of the model
+ * snapshot at the rows of a sub-block step (modeling.py:153-166, :325).
+ * ------------------------------------------------------------------------- */
+int fdllm_linear_workspace_size(int rows, int out_features, int in_features, int gated, size_t* bytes);
+int fdllm_linear(const void* x, int64_t x_stride_row, const void* w, const void* w_up, const void* bias, void* out,
+                 int rows, int out_features, int in_features, int dtype, void* workspace, size_t workspace_bytes,
+                 void* stream);
+
 /* -------------------------------------------------------------------------
  * One greedy sampling + threshold unmasking step of a sub-block.
  *

@@ -1,0 +1,100 @@
+"""ops.linear / ops.gated_linear (fdllm_linear) and the few-row form of
+ops.qkv_rope_kv_write against torch in float64."""
+import pytest
+import torch
+
+from fast_v2_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _ints(gen, *shape, dtype):
+    """Small whole numbers: every fp32 sum of up to 2^20 products of them is exact, in any
+    order, so results compare bit for bit."""
+    return torch.randint(-3, 4, shape, generator=gen, device="cuda").to(dtype)
+
+
+# rows at the edges of the 16-row MFMA tile counts; columns and K where a layer is one
+# tile, a partial last tile, tiles cut evenly (<= 128 tiles) and ranges that cross tiles
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 64, 65, 128])
+@pytest.mark.parametrize("n,k", [(8, 64), (72, 576), (200, 4096), (8320, 1088), (16648, 192)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_exact(gpu, m, n, k, dtype):
+    print(f"case linear {m}x{n}x{k} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + n)
+    x, w, b = _ints(g, m, k, dtype=dtype), _ints(g, n, k, dtype=dtype), _ints(g, n, dtype=dtype)
+    want = x.double() @ w.double().t().contiguous()
+    for bias in (None, b):
+        ref = want if bias is None else want + b.double()
+        for _ in range(2):  # the arrival counters are back at zero after a call
+            got = ops.linear(x, w, bias)
+            assert torch.equal(got, ref.float().to(dtype))
+
+
+def test_linear_strided_rows(gpu):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    full = _ints(g, 40, 2, 256, dtype=torch.bfloat16)
+    w = _ints(g, 128, 256, dtype=torch.bfloat16)
+    for x in (full[:, 1], full[:, 1, :][::2], full.view(40, 512)[:, 8:264], full.view(40, 512)[:, 1:257]):
+        assert torch.equal(ops.linear(x, w), (x.double() @ w.double().t().contiguous()).float().to(x.dtype))
+
+
+@pytest.mark.parametrize("m", [1, 31, 128])
+@pytest.mark.parametrize("n,k", [(8, 64), (104, 1536), (4360, 1088)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gated_linear(gpu, m, n, k, dtype):
+    print(f"case gated {m}x{n}x{k} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    x, wg, wu = _ints(g, m, k, dtype=dtype), _ints(g, n, k, dtype=dtype), _ints(g, n, k, dtype=dtype)
+    wg = wg * 0.015625  # exact, and gates of a few units instead of saturated ones
+    gate, up = ((x.double() @ w.double().t().contiguous()).float().to(dtype) for w in (wg, wu))
+    want = ops.silu_mul(gate, up)
+    assert torch.equal(ops.gated_linear(x, wg, wu), want)
+
+
+def test_linear_graph_replay(gpu):
+    """Partial sums and counters under graph replay, with other calls in between."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, w = _ints(g, 24, 4096, dtype=torch.bfloat16), _ints(g, 200, 4096, dtype=torch.bfloat16)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        ops.linear(x, w)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            out = ops.linear(x, w)
+        for i in range(4):
+            x.copy_(_ints(g, 24, 4096, dtype=torch.bfloat16))
+            graph.replay()
+            assert torch.equal(out, ops.linear(x, w))
+            assert torch.equal(out, (x.double() @ w.double().t().contiguous()).float().to(x.dtype))
+            s.synchronize()
+
+
+@pytest.mark.parametrize("bad", ["rows", "k", "n", "dtype", "grad"])
+def test_linear_refuses(gpu, bad):
+    x = torch.zeros(129 if bad == "rows" else 8, 96 if bad == "k" else 128, device="cuda", dtype=torch.bfloat16)
+    w = torch.zeros(12 if bad == "n" else 16, x.shape[1], device="cuda",
+                    dtype=torch.float16 if bad == "dtype" else torch.bfloat16, requires_grad=bad == "grad")
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w)
+
+
+@pytest.mark.parametrize("rows", [(1, 1), (4, 8), (5, 13), (4, 32)])
+def test_qkv_linear_is_the_fused_kernels_projection(gpu, rows):
+    """Plain projections, and the ones that qkv_rope_kv_write rotates (v rows as they are)."""
+    g = torch.Generator(device="cuda").manual_seed(11)
+    b, s = rows
+    dt = torch.bfloat16
+    x = torch.randn(b, s, 1536, generator=g, device="cuda").to(dt)
+    w = [(torch.randn(n, 1536, generator=g, device="cuda") * 0.02).to(dt) for n in (768, 256, 256)]
+    bias = [torch.randn(t.shape[0], generator=g, device="cuda").to(dt) for t in w]
+    args = [t for pair in zip(w, bias) for t in pair]
+    q, k, v = ops.qkv_linear(x, *args)
+    for got, wt, bt in zip((q, k, v), w, bias):
+        want = x.double() @ wt.double().t().contiguous() + bt.double()
+        # one rounding to bf16 (half of 2^-7 of the value) and fp32 sums of 1536 products
+        torch.testing.assert_close(got.reshape(b, s, -1).double(), want, rtol=2.0 ** -8 + 2e-5, atol=2e-4)
+    cos, sin = (torch.randn(1, s, 128, generator=g, device="cuda").to(dt) for _ in range(2))
+    q_rot, (k_rot, v_out) = ops.qkv_rope_kv_write(x, *args, cos, sin, kv_out=True)
+    q2, (k2, v2) = ops.rope_kv_write(q, k, v, cos, sin, kv_out=True)
+    assert torch.equal(q_rot, q2) and torch.equal(k_rot, k2) and torch.equal(v_out, v2) and torch.equal(v, v2)

@@ -1,0 +1,34 @@
+"""Which linear layers the weight-streaming kernels may stand in for (no GPU needed: the
+rule refuses before any launch)."""
+import torch
+import torch.nn as nn
+import torch.nn.utils.parametrize as parametrize
+
+from fast_v2_amd import ops
+from fast_v2_amd.utils import linear_layers as ll
+
+
+class _Adapted(nn.Linear):
+    pass
+
+
+def test_only_plain_layers():
+    lin = nn.Linear(64, 8)
+    assert ll.plain_linear(lin)
+    h = lin.register_forward_hook(lambda m, a, o: o + 1)
+    assert not ll.plain_linear(lin)
+    h.remove()
+    assert ll.plain_linear(lin)
+    lin.forward = lambda x: x
+    assert not ll.plain_linear(lin)
+    assert not ll.plain_linear(_Adapted(64, 8))
+    par = nn.Linear(64, 8)
+    parametrize.register_parametrization(par, "weight", nn.Identity())
+    assert not ll.plain_linear(par)
+
+
+def test_project_runs_the_module_on_cpu():
+    lin = nn.Linear(64, 8).to(torch.bfloat16)
+    x = torch.randn(3, 64).to(torch.bfloat16)
+    assert not ll.streams(x, lin) and not ops.linear_fits(x, lin.weight)
+    assert torch.equal(ll.project(lin, x), lin(x))
