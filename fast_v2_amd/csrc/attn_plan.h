@@ -53,6 +53,9 @@ constexpr int kF32TargetWG = 512;
 #endif
 constexpr int kF32MaxSplits = 16;      // fp32 kernel: key splits per row block at most
 constexpr size_t kCounterBytes = 64 * 1024;  // arrival counters at the head of the workspace
+// bytes of the library's scratch (fdllm_kv_attn_fwd_noalloc) behind the counters, less the
+// rounding of the (m, l) region
+constexpr int64_t kScratchSlotBytes = FDLLM_KV_ATTN_SCRATCH_BYTES - kCounterBytes - 4096;
 constexpr uint32_t kMaxGridX = 0x7fffffffu;  // grid limits of a launch
 constexpr uint32_t kMaxGridYZ = 65535u;
 
@@ -204,7 +207,15 @@ inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl) {
       }
       if (d->kv_split == 0 && B <= kBalancedMaxBatch) {
         pl->chunk = 0;
-        slots = std::max<int64_t>((kDecodeSlotsTarget + hkv - 1) / hkv, B * min_splits);
+        // one workgroup per compute unit, or whole multiples of that where long sequences may
+        // need more: 16-bit 28 / 4 heads, token-major pages, 24 x 2000-12000 keys 98.6 us
+        // with 72 slots, 79.0 with 128; 40 x 2000-6000 90.4 with 80, 73.8 with 128; 48 x
+        // 2000-6000 98.0 with 96, 87.4 with 128. More rounds than needed only cost (16 x
+        // 2000-6000: 33 us with 64 slots, 43 with 128).
+        const int64_t round = (kDecodeSlotsTarget + hkv - 1) / hkv;
+        slots = std::max<int64_t>(round, (B * min_splits + round - 1) / round * round);
+        // (what the library's scratch holds without the rounding keeps fitting it)
+        if (slots * hkv * 64 * (d->head_dim + 2) * 4 > kScratchSlotBytes) slots = std::max(round, B * min_splits);
         pl->n_splits = static_cast<int>(slots);
         split_possible = slots > B;
       } else {
