@@ -75,6 +75,7 @@ enum PlanKind {
 
 struct Plan {
   int kind;     // PlanKind
+  bool ring;    // general plan run by the ring prefill kernel (plan_ring_chunk)
   bool decode;  // all-heads decode kernel (kv_decode_kernel)
   int MT, rows_per_wg, n_rb, n_splits, chunk, R;
   size_t ws_o_bytes, ws_ml_bytes;
@@ -87,12 +88,64 @@ inline int64_t plan_max_keys(const fdllm_kv_attn_desc* d) {
                        : d->max_seqlen;
 }
 
+// Key ranges of the ring prefill kernel where the row blocks of 256 rows leave compute units
+// idle: the splits of the longest block (1: none) and the 64-key tiles per split. Such a
+// call lasts as long as its longest workgroup, 12.5 us and 1.3 us per tile; ranges that
+// still fit one workgroup per compute unit shorten that and cost their partials, 2.5 us and
+// 0.053 us per workgroup (fitted to 12-2 and 28-4 heads, 40-3000 tokens after up to 2048).
+// Lengths are taken at the cache's capacity (the host knows no others): at shorter ones the
+// kernel cuts less, never wrongly. Bounded by the library's scratch, so that calls without a
+// workspace of their own stay possible. Measured, us (start: the general kernel up to 2047
+// rows, whole ranges above): 1 x 500 tokens after 2048, 28/4 heads, 64.7 -> 40.3; 1 x 1000
+// after 1024 55.9 -> 47; 1 x 40 after 2048 29.6 -> 22.9; 12/2 heads, block-causal, 1 x 3000
+// 74.8 -> 51, 1 x 2000 50.7 -> 36; 1 x 1500 of 28/4 heads stays whole (42, two ranges 40).
+inline void plan_ring_chunk(const fdllm_kv_attn_desc* d, int R, int64_t max_len, int64_t* splits, int64_t* chunk_tiles) {
+  const int G = d->num_q_heads / d->num_kv_heads;
+  const int n_rb = (R + 255) / 256;
+  const int64_t bh = static_cast<int64_t>(std::max(d->batch, 1)) * d->num_kv_heads;
+  const int64_t max_t = std::max<int64_t>(1, (max_len + 63) / 64);
+  *splits = 1;
+  *chunk_tiles = max_t;
+  if (bh * n_rb > 256) return;
+  const int64_t fit = kScratchSlotBytes / (bh * n_rb * 256 * (128 + 2) * 4);
+  double best = 0;
+  int64_t last = 0;
+  for (int64_t n = 1; n <= std::min<int64_t>(fit, kMaxDecodeSplits) || n == 1; ++n) {
+    const int64_t c = (max_t + n - 1) / n;
+    if (n > 1 && (c == last || c < 4)) continue;
+    last = c;
+    int64_t wgs = 0, longest = 0;
+    for (int rb = 0; rb < n_rb; ++rb) {
+      const int64_t pos = max_len - d->q_len + (std::min(R, (rb + 1) * 256) - 1) / G;  // last row's position
+      int64_t end = max_len;
+      if (d->mask_mode == FDLLM_MASK_CAUSAL) end = pos + 1;
+      else if (d->mask_mode == FDLLM_MASK_BLOCK_CAUSAL) end = (pos / d->mask_block + 1) * d->mask_block;
+      const int64_t t = (std::max<int64_t>(0, std::min(end, max_len)) + 63) / 64;
+      const int64_t k = std::max<int64_t>(1, (t + c - 1) / c);
+      wgs += k;
+      longest = std::max(longest, (t + k - 1) / k);
+    }
+    if (n > 1 && wgs * bh > kSplitTargetWG) continue;
+    // in tiles; one tile of margin against the fit, and slower tiles with nearly every
+    // compute unit busy
+    const double w = static_cast<double>(wgs * bh);
+    const double cost = n > 1 ? static_cast<double>(longest) * std::max(1.0, w / 210) + 2.9 + 0.041 * w
+                              : static_cast<double>(longest);
+    if (n == 1 || cost < best) {
+      best = cost;
+      *chunk_tiles = c;
+      *splits = (max_t + c - 1) / c;
+    }
+  }
+}
+
 // Split-KV decode: by default the kernel partitions the keys itself from the device-side
 // lengths over S slots per KV head (S * Hkv ~ one workgroup per CU); a caller-given
 // kv_split fixes the keys per split instead.
 inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl) {
   FDLLM_CHECK_ARG(d != nullptr, "fdllm_kv_attn: null descriptor");
   pl->ws_unit_off = 0;
+  pl->ring = false;
   FDLLM_CHECK_ARG(d->dtype == FDLLM_DTYPE_BF16 || d->dtype == FDLLM_DTYPE_F16 || d->dtype == FDLLM_DTYPE_F32,
                   "fdllm_kv_attn: dtype %d unsupported (bf16, fp16 or fp32)", d->dtype);
   FDLLM_CHECK_ARG(d->head_dim == 64 || d->head_dim == 128, "fdllm_kv_attn: head_dim %d unsupported (64 or 128)",
@@ -315,7 +368,19 @@ inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl) {
                              pl->R >= 8 * 256 && d->kv_split == 0 &&
                              (d->page_table == nullptr || d->page_size >= 32) && d->k_stride_slot < (1 << 24) &&
                              d->v_stride_slot < (1 << 24) && (pl->R + 255) / 256 < 65536;
-  if (prefill_shape) {
+  // ... or fewer rows, or key ranges to be cut: the general plan's fixed key chunks on the
+  // ring kernel (whole rows of every stride it takes lie within its buffer descriptors).
+  // 257 to 2047 rows, 28/4 heads: 2 x 157 tokens 15.0 us against 20.7 in the general kernel,
+  // 1 x 290 18.1 against 27.3, 16 x 157 26 against 42.5
+  const bool ring_shape = !(d->flags & FDLLM_ATTN_NO_DECODE_KERNEL) && d->head_dim == 128 && pl->R > 256 &&
+                          d->kv_split == 0 && (d->page_table == nullptr || (d->page_size >= 32 && max_len <= 65152)) &&
+                          d->k_stride_slot >= 128 && d->v_stride_slot >= 128 && d->k_stride_slot < (1 << 24) &&
+                          d->v_stride_slot < (1 << 24) && (pl->R + 255) / 256 < 65536 &&
+                          (d->k_new == nullptr || d->new_stride_s >= 128);
+  int64_t ring_splits = 1, ring_tiles = 1;
+  if (ring_shape) plan_ring_chunk(d, pl->R, max_len, &ring_splits, &ring_tiles);
+  pl->ring = ring_shape && (ring_splits > 1 || !prefill_shape);
+  if (prefill_shape && !pl->ring) {
     pl->kind = kPlanPrefill;
     pl->MT = 4;
     pl->rows_per_wg = 32 * kPrefillWaves;
@@ -326,13 +391,15 @@ inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl) {
     return FDLLM_OK;
   }
   const int mtiles = (pl->R + 15) / 16;
-  pl->MT = mtiles <= 4 ? 1 : (mtiles <= 8 ? 2 : 4);
+  pl->MT = mtiles <= 4 ? 1 : (mtiles <= 8 ? 2 : 4);  // 4 (256 rows) where the ring kernel runs it
   pl->rows_per_wg = 64 * pl->MT;
   pl->n_rb = (pl->R + pl->rows_per_wg - 1) / pl->rows_per_wg;
   const int64_t max_tiles = std::max<int64_t>(1, (max_len + kKT - 1) / kKT);
   int64_t chunk_tiles;
   const int64_t units = static_cast<int64_t>(d->batch) * d->num_kv_heads * pl->n_rb;
-  if (d->kv_split > 0) {
+  if (pl->ring) {
+    chunk_tiles = ring_tiles;
+  } else if (d->kv_split > 0) {
     chunk_tiles = d->kv_split / kKT;
   } else {
     // Aim for ~2 workgroups per CU (256 CUs) when every sequence is full length.
@@ -373,7 +440,7 @@ inline size_t plan_workspace_bytes(const fdllm_kv_attn_desc*, const Plan& pl) {
 }
 
 // The rows of k_new / v_new are stored from inside the prefill kernels (plan kinds
-// prefill and split prefill, no explicit q_start, no FDLLM_ATTN_CACHE_WRITE_KERNEL);
+// prefill and split prefill, and general on the ring kernel; no explicit q_start, no FDLLM_ATTN_CACHE_WRITE_KERNEL);
 // otherwise a copy kernel stores them ahead of the attention.
 // The prefill kernels read every key at or past the query start from the new rows,
 // which is exact only when no visible key lies past the last new row. Without q_start
@@ -382,7 +449,7 @@ inline size_t plan_workspace_bytes(const fdllm_kv_attn_desc*, const Plan& pl) {
 // copy kernel, which stores the rows before the attention reads the cache.
 inline bool plan_fuses_cache_write(const fdllm_kv_attn_desc* d, const Plan& pl) {
   return d->k_new != nullptr && d->q_start == nullptr && !(d->flags & FDLLM_ATTN_CACHE_WRITE_KERNEL) &&
-         (pl.kind == kPlanPrefill || pl.kind == kPlanSplitPrefill);
+         (pl.kind == kPlanPrefill || pl.kind == kPlanSplitPrefill || pl.ring);
 }
 
 // The fp32 plan merges its key splits in the kernel (one counter per row block unit).

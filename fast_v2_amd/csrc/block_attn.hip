@@ -2150,8 +2150,9 @@ __global__ __launch_bounds__(256) void kv_attn_f32_kernel(const AttnParams p) {
 // agreement fell from 0.8721 / 0.8751 to 0.8700 / 0.8724 against a noise floor of 0.8739,
 // s.e. 0.0013, as with bf16 rows: the extra rounding of every split moves near-tied
 // greedy choices), so the rows stay fp32.
-__device__ __forceinline__ void split_prefill_partial(const AttnParams& p, int64_t slot0, int split, int r, int h,
-                                                      const f32x16 (&acc)[4], float m_run, float l_run) {
+// rl: the row's place in its row block.
+__device__ __forceinline__ void split_prefill_partial(const AttnParams& p, int64_t slot0, int split, int r, int rl,
+                                                      int h, const f32x16 (&acc)[4], float m_run, float l_run) {
   constexpr int D = 128;
   if (r < p.R) {
     const int64_t slot = slot0 + split;
@@ -2162,10 +2163,10 @@ __device__ __forceinline__ void split_prefill_partial(const AttnParams& p, int64
       for (int i = 0; i < 4; ++i)
         __builtin_amdgcn_raw_buffer_store_b128(
             __builtin_bit_cast(u32x4, f32x4{acc[dt][4 * i], acc[dt][4 * i + 1], acc[dt][4 * i + 2], acc[dt][4 * i + 3]}),
-            orsrc, (r * D + 32 * dt + 8 * i + 4 * h) * 4, 0, 0);
+            orsrc, (rl * D + 32 * dt + 8 * i + 4 * h) * 4, 0, 0);
     if (h == 0) {
       const auto mrsrc = __builtin_amdgcn_make_buffer_rsrc(p.ws_ml + slot * 256, 0, 256 * 8, kBufferFlags);
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, make_float2(m_run, l_run)), mrsrc, r * 8, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, make_float2(m_run, l_run)), mrsrc, rl * 8, 0, 0);
     }
   }
 }
@@ -2648,7 +2649,7 @@ __global__ __launch_bounds__(64 * NW, 2) void kv_prefill_kernel(FDLLM_LEAD_PARAM
     // which the merge kernel then skips (its entry must not be left from an earlier call)
     if (split == 0 && tid == 0 && p.ws_unit != nullptr) p.ws_unit[b * p.Hkv + kvh] = make_int2(first, n_act);
     if (n_act > 1) {
-      split_prefill_partial(p, first, split, r, h, acc, m_run, l_run);
+      split_prefill_partial(p, first, split, r, r, h, acc, m_run, l_run);
       return;
     }
   }
@@ -2706,9 +2707,21 @@ constexpr int kRingMaxHalves = 2048;
 //     are avoided by an XOR swizzle of the 16-byte chunks, applied on the source
 //     side: LDS chunk p of K row r holds column chunk p ^ (r & 15), of V row r
 //     chunk p ^ 4 (r & 3).
-template <bool F16, bool PAGED, bool SPLIT, bool FUSED>
+//   * Key ranges (MODE). Whole: one workgroup per row block. Sequence: one row block per
+//     (sequence, KV head), keys dealt by decode_partition. Chunk: row blocks whose keys are
+//     cut into equal ranges of at most p.chunk keys, partials laid out as the general
+//     kernel's and folded by kv_attn_combine_kernel. Workgroups are numbered by range, then
+//     longest row block first, then (sequence, KV head): the ranges that short row blocks
+//     do not have come last, so the working ones are dealt evenly to the XCDs (numbered row
+//     block by row block, the working ranges of short blocks fell on two of the eight: 1 x
+//     2000 tokens of 12 / 2 heads in four ranges took 50.7 us, two 37.6).
+enum RingMode { kRingWhole = 0, kRingSequence = 1, kRingChunk = 2 };
+
+template <bool F16, bool PAGED, int MODE, bool FUSED>
 __global__ __launch_bounds__(512, 2) void kv_prefill_ring_kernel(FDLLM_LEAD_PARAMS, const AttnParams p) {
   FDLLM_LEAD_LOCAL;
+  constexpr bool SPLIT = MODE == kRingSequence;
+  constexpr bool CHUNK = MODE == kRingChunk;
   FDLLM_STAMP(0, __builtin_amdgcn_s_memrealtime());  // start
   constexpr int D = 128;
   constexpr int KT = 64;
@@ -2746,6 +2759,24 @@ __global__ __launch_bounds__(512, 2) void kv_prefill_ring_kernel(FDLLM_LEAD_PARA
     si.seqlen = dp.seqlen;
     si.qs = dp.qs;
     si.kv_end = dp.kv_end;
+  } else if constexpr (CHUNK) {
+    const int id = static_cast<int>(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+    const int pairs = p.B * p.Hkv;
+    const int rest = id / pairs;
+    const int bh = id - rest * pairs;
+    split = rest / p.n_rb;
+    const int back = rest - split * p.n_rb;  // row blocks from the last
+    b = bh / p.Hkv;
+    kvh = bh - b * p.Hkv;
+    rb = p.n_rb - 1 - back;
+    si = seq_info<PAGED>(p, ld, b, rb);
+    n_act = max(1, si.n_act);
+    if (split >= n_act) return;  // uniform over the workgroup
+    first = (bh * p.n_rb + rb) * p.n_splits;
+    const int tiles = (si.kv_end + KT - 1) / KT;
+    const int size = (tiles + n_act - 1) / n_act * KT;
+    k_lo = __builtin_amdgcn_readfirstlane(min(split * size, si.kv_end));
+    k_hi = __builtin_amdgcn_readfirstlane(min(si.kv_end, k_lo + size));
   } else {
     const int unit = blockIdx.x;
     b = unit / p.Hkv;
@@ -2771,6 +2802,7 @@ __global__ __launch_bounds__(512, 2) void kv_prefill_ring_kernel(FDLLM_LEAD_PARA
     } else {
       w_lo = qs + (256 * rb) / p.G;
       w_hi = qs + min(p.Sq, (256 * (rb + 1)) / p.G);
+      if (split != 0) w_hi = w_lo;  // the row block's first key range stores them
     }
     w_lo = __builtin_amdgcn_readfirstlane(max(w_lo, 0));
     w_hi = __builtin_amdgcn_readfirstlane(min(w_hi, p.cap));
@@ -2793,7 +2825,11 @@ __global__ __launch_bounds__(512, 2) void kv_prefill_ring_kernel(FDLLM_LEAD_PARA
           ? INT_MIN
           : __builtin_amdgcn_readfirstlane(static_cast<int>(wave_allreduce_max(static_cast<float>(lim))));
   const float c2 = p.scale_log2;
-  const float rescale_thr = 8.f / c2;
+  // Chunk: below the whole-range form's 2048 rows the reference follows every new maximum, so
+  // that a row's largest probability is 1 exactly, as in the general kernel, whose shapes
+  // those are (2 x 157 tokens, distance from 64-bit results 0.0021, 0.0023 with the lazy
+  // reference; 1 x 290 tokens 19.6 us against 18.3)
+  const float rescale_thr = CHUNK && p.R < 2048 ? 0.f : 8.f / c2;
 
   f32x16 acc[4];
 #pragma unroll
@@ -3329,8 +3365,14 @@ __global__ __launch_bounds__(512, 2) void kv_prefill_ring_kernel(FDLLM_LEAD_PARA
     // which the merge kernel then skips (its entry must not be left from an earlier call)
     if (split == 0 && tid == 0 && p.ws_unit != nullptr) p.ws_unit[b * p.Hkv + kvh] = make_int2(first, n_act);
     if (n_act > 1) {
-      split_prefill_partial(p, first, split, r, h, acc, m_run, l_run);
+      split_prefill_partial(p, first, split, r, r, h, acc, m_run, l_run);
       FDLLM_STAMP(4, __builtin_amdgcn_s_memrealtime());  // partial stores issued
+      return;
+    }
+  }
+  if constexpr (CHUNK) {
+    if (n_act > 1) {
+      split_prefill_partial(p, first, split, r, r - row0, h, acc, m_run, l_run);
       return;
     }
   }
@@ -3512,6 +3554,18 @@ void launch_combine(const AttnParams& p, dim3 cgrid, hipStream_t s) {
 #ifndef FDLLM_PREFILL_RING
 #define FDLLM_PREFILL_RING 1
 #endif
+template <int MODE, bool FUSED>
+void launch_ring(const AttnParams& p, bool f16, dim3 grid, hipStream_t s) {
+  const bool paged = p.page_table != nullptr;
+  if (f16) {
+    if (paged) kv_prefill_ring_kernel<true, true, MODE, FUSED><<<grid, dim3(512), 0, s>>>(FDLLM_LEAD_ARGS(p), p);
+    else kv_prefill_ring_kernel<true, false, MODE, FUSED><<<grid, dim3(512), 0, s>>>(FDLLM_LEAD_ARGS(p), p);
+  } else {
+    if (paged) kv_prefill_ring_kernel<false, true, MODE, FUSED><<<grid, dim3(512), 0, s>>>(FDLLM_LEAD_ARGS(p), p);
+    else kv_prefill_ring_kernel<false, false, MODE, FUSED><<<grid, dim3(512), 0, s>>>(FDLLM_LEAD_ARGS(p), p);
+  }
+}
+
 template <bool SPLIT, bool FUSED>
 void launch_prefill(const AttnParams& p, bool f16, dim3 grid, hipStream_t s) {
   constexpr int NW = SPLIT ? 8 : kPrefillWaves;
@@ -3521,13 +3575,7 @@ void launch_prefill(const AttnParams& p, bool f16, dim3 grid, hipStream_t s) {
                                  : p.max_seqlen;
   if (FDLLM_PREFILL_RING && (!SPLIT || FDLLM_PREFILL_RING_SPLIT) &&
       (!paged || max_keys + 6 * 64 <= static_cast<int64_t>(kRingMaxHalves) * 32)) {
-    if (f16) {
-      if (paged) kv_prefill_ring_kernel<true, true, SPLIT, FUSED><<<grid, dim3(512), 0, s>>>(FDLLM_LEAD_ARGS(p), p);
-      else kv_prefill_ring_kernel<true, false, SPLIT, FUSED><<<grid, dim3(512), 0, s>>>(FDLLM_LEAD_ARGS(p), p);
-    } else {
-      if (paged) kv_prefill_ring_kernel<false, true, SPLIT, FUSED><<<grid, dim3(512), 0, s>>>(FDLLM_LEAD_ARGS(p), p);
-      else kv_prefill_ring_kernel<false, false, SPLIT, FUSED><<<grid, dim3(512), 0, s>>>(FDLLM_LEAD_ARGS(p), p);
-    }
+    launch_ring<SPLIT ? kRingSequence : kRingWhole, FUSED>(p, f16, grid, s);
     return;
   }
   if (f16) {
@@ -3560,6 +3608,17 @@ void launch_decode(const AttnParams& p, bool f16, const LaunchSet& ls, hipStream
       if (paged) launch_combine<128, false, true>(p, cgrid, s);
       else launch_combine<128, false, false>(p, cgrid, s);
     }
+  }
+}
+
+void launch_combine_16(const AttnParams& p, bool f16, dim3 grid, hipStream_t s) {
+  const bool paged = p.page_table != nullptr;
+  if (f16) {
+    if (paged) launch_combine<128, true, true>(p, grid, s);
+    else launch_combine<128, true, false>(p, grid, s);
+  } else {
+    if (paged) launch_combine<128, false, true>(p, grid, s);
+    else launch_combine<128, false, false>(p, grid, s);
   }
 }
 
@@ -3792,6 +3851,13 @@ int kv_attn_launch(const fdllm_kv_attn_desc* d, const Plan& pl, void* workspace,
       if (f16) kv_split_prefill_merge_kernel<true><<<mgrid, dim3(256), 0, s>>>(p);
       else kv_split_prefill_merge_kernel<false><<<mgrid, dim3(256), 0, s>>>(p);
     }
+    FDLLM_RETURN_LAUNCH_STATUS("fdllm_kv_attn_fwd");
+  }
+  if (pl.ring) {
+    const dim3 grid = to_dim3(ls.main_grid);
+    if (fuse_write) launch_ring<kRingChunk, true>(p, f16, grid, s);
+    else launch_ring<kRingChunk, false>(p, f16, grid, s);
+    if (ls.second) launch_combine_16(p, f16, to_dim3(ls.second_grid), s);
     FDLLM_RETURN_LAUNCH_STATUS("fdllm_kv_attn_fwd");
   }
   if (pl.decode) {

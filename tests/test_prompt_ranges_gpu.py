@@ -1,0 +1,111 @@
+"""Prompts of few row blocks: the ring prefill kernel with and without key ranges against
+float64 and against the general kernel (decode_kernel=False) over the forms it takes."""
+import itertools
+
+import pytest
+import torch
+
+from fast_v2_amd import _ffi, ops
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _case(b, sq, heads, cap, layout, dtype, seed):
+    hq, hkv = heads
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g, device="cuda").to(dtype)
+    q = rnd(b, sq, hq, D)
+    if layout == "contiguous":
+        k, v, table = rnd(b, cap, hkv, D), rnd(b, cap, hkv, D), None
+    else:
+        pages = (cap + 31) // 32
+        k, v = rnd(b * pages, 32, hkv, D), rnd(b * pages, 32, hkv, D)
+        if layout == "paged_hm":
+            k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (k, v))
+        table = torch.randperm(b * pages, generator=g, device="cuda").to(torch.int32).view(b, pages)
+    return q, k, v, table, rnd(b, sq, hkv, D), rnd(b, sq, hkv, D)
+
+
+def _dense(t, table, b):
+    return t[b] if table is None else t[table[b].long()].flatten(0, 1)
+
+
+def _ref(q, k, v, table, lens, starts, mode, block=32):
+    out = torch.zeros(q.shape, dtype=torch.float64, device="cuda")
+    b, sq, hq, _ = q.shape
+    for i in range(b):
+        kk, vv = (_dense(t, table, i).double() for t in (k, v))
+        pos = starts[i] + torch.arange(sq, device="cuda")
+        lim = torch.full_like(pos, lens[i])
+        if mode == _ffi.MASK_CAUSAL:
+            lim = torch.minimum(lim, pos + 1)
+        elif mode == _ffi.MASK_BLOCK_CAUSAL:
+            lim = torch.minimum(lim, torch.where(pos >= 0, (pos // block + 1) * block, torch.zeros_like(pos)))
+        hide = torch.arange(kk.shape[0], device="cuda")[None] >= lim[:, None]
+        for h in range(hq):
+            g = h // (hq // kk.shape[1])
+            s = (q[i, :, h].double() @ kk[:, g].t().contiguous() * D ** -0.5).masked_fill(hide, float("-inf"))
+            p = torch.nan_to_num(torch.softmax(s, dim=-1))  # a row that sees no key is zero
+            out[i, :, h] = p @ vv[:, g].contiguous()
+    return out
+
+
+# rows per KV head: 259 (two row blocks), 1099, 2037 / 2051 (around the whole-range form's
+# start), 3500; key ranges where the capacity is long; visible lengths at, below and far
+# below the capacity (one sequence empty of keys to range over)
+SHAPES = [(1, 37, (28, 4), 37), (2, 157, (28, 4), 157), (1, 291, (28, 4), 1500), (1, 293, (28, 4), 293),
+          (1, 500, (28, 4), 1203), (1, 300, (12, 2), 2048), (3, 70, (12, 2), 700), (1, 129, (2, 1), 4096)]
+
+
+@pytest.mark.parametrize("b,sq,heads,cap", SHAPES)
+@pytest.mark.parametrize("mode", [_ffi.MASK_SEQLEN, _ffi.MASK_CAUSAL, _ffi.MASK_BLOCK_CAUSAL])
+@pytest.mark.parametrize("layout", ["contiguous", "paged", "paged_hm"])
+def test_prompt(gpu, b, sq, heads, cap, mode, layout):
+    dtype = torch.float16 if layout == "paged" else torch.bfloat16
+    q, k, v, table, kn, vn = _case(b, sq, heads, cap, layout, dtype, cap + sq + mode)
+    kw = dict(mask_mode=mode, page_table=table, page_size=32 if table is not None else 0)
+    for short, write in itertools.product((False, True), (False, True)):
+        lens = [max(sq, cap - 65 * i - (cap // 2 if short else 0)) for i in range(b)]
+        seqlens = torch.tensor(lens, dtype=torch.int32, device="cuda")
+        print(f"case prompt {b}x{sq} {heads} cap {cap} mode {mode} {layout} lens {lens} write {write}", flush=True)
+        ka, va, kb, vb = k.clone(), v.clone(), k.clone(), v.clone()
+        new = dict(k_new=kn, v_new=vn) if write else {}
+        got = ops.block_attn(q, ka, va, seqlens, **kw, **new)
+        gen = ops.block_attn(q, kb, vb, seqlens, decode_kernel=False, **kw, **new)
+        assert torch.equal(ka, kb) and torch.equal(va, vb)
+        want = _ref(q, ka, va, table, lens, [n - sq for n in lens], mode)
+        # probabilities and results are rounded to the type once each
+        torch.testing.assert_close(got.double(), want, atol=1e-2, rtol=1e-2)
+        torch.testing.assert_close(gen.double(), want, atol=1e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("starts", [[0, 400], [-20, 100]])
+def test_prompt_query_starts_and_empty_rows(gpu, starts):
+    q, k, v, table, kn, vn = _case(2, 150, (28, 4), 640, "paged", torch.bfloat16, 5)
+    qs = torch.tensor(starts, dtype=torch.int32, device="cuda")
+    for lens in ([640, 555], [0, 31]):
+        seqlens = torch.tensor(lens, dtype=torch.int32, device="cuda")
+        for mode in (_ffi.MASK_SEQLEN, _ffi.MASK_CAUSAL, _ffi.MASK_BLOCK_CAUSAL):
+            print(f"case starts {starts} lens {lens} mode {mode}", flush=True)
+            got = ops.block_attn(q, k, v, seqlens, mask_mode=mode, q_start=qs, page_table=table, page_size=32)
+            torch.testing.assert_close(got.double(), _ref(q, k, v, table, lens, starts, mode), atol=1e-2, rtol=1e-2)
+
+
+def test_prompt_graph_replay(gpu):
+    """Ranges and their merge under graph replay with eager calls in between."""
+    q, k, v, table, kn, vn = _case(1, 500, (28, 4), 1203, "contiguous", torch.bfloat16, 9)
+    seqlens = torch.tensor([1203], dtype=torch.int32, device="cuda")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        ops.block_attn(q, k, v, seqlens, mask_mode=_ffi.MASK_CAUSAL)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            out = ops.block_attn(q, k, v, seqlens, mask_mode=_ffi.MASK_CAUSAL)
+        for n in (1203, 900, 500):
+            seqlens.fill_(n)
+            graph.replay()
+            assert torch.equal(out, ops.block_attn(q, k, v, seqlens, mask_mode=_ffi.MASK_CAUSAL))
+            s.synchronize()
