@@ -31,7 +31,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import _ffi, ops
-from .linear_layers import project, streams
+from .linear_layers import streams
 from .static_kv_cache import StaticKVCache
 
 logger = logging.getLogger(__name__)
@@ -264,9 +264,6 @@ def _create_patched_attention_forward(attn_module, attn_backend, static_block_ca
                                     replace_position, **kwargs)
         input_shape = hidden_states.shape[:-1]
         hidden_shape = (*input_shape, -1, head_dim)
-
-        def o_proj(x):
-            return project(attn_module.o_proj, x) if getattr(attn_module, "fused", False) else attn_module.o_proj(x)
         cos, sin = position_embeddings
         fused = attn_backend.name == AttentionBackend.HIP and FUSED_ROPE_CACHE_WRITE
         rope_ok, proj_ok = _fusable(attn_module, hidden_states, head_dim) if fused else (False, False)
@@ -283,7 +280,7 @@ def _create_patched_attention_forward(attn_module, attn_backend, static_block_ca
                 out = attn_backend.flash_kvcache_attention(q, full_k, full_v,
                                                            cache_seqlens=past_key_value.scratch_seqlens,
                                                            is_causal=False, scaling=scaling)
-                return o_proj(out.reshape(*input_shape, -1))
+                return attn_module.o_proj(out.reshape(*input_shape, -1))
         if few:  # the same projections as above, bit for bit
             q, k, v = ops.qkv_linear(hidden_states, qp.weight, qp.bias, kp.weight, kp.bias, vp.weight, vp.bias,
                                      head_dim)
@@ -302,7 +299,7 @@ def _create_patched_attention_forward(attn_module, attn_backend, static_block_ca
                 out = attn_backend.flash_kvcache_attention(q_rot, full_k, full_v,
                                                            cache_seqlens=past_key_value.scratch_seqlens,
                                                            is_causal=False, scaling=scaling)
-                return o_proj(out.reshape(*input_shape, -1))
+                return attn_module.o_proj(out.reshape(*input_shape, -1))
         q, k = _apply_rotary_pos_emb(q, k, cos, sin)
 
         if block_past_key_values is not None:
@@ -325,7 +322,7 @@ def _create_patched_attention_forward(attn_module, attn_backend, static_block_ca
         out = attn_backend.flash_kvcache_attention(q, full_k, full_v, cache_seqlens=past_key_value.scratch_seqlens,
                                                    is_causal=False, scaling=scaling)
         out = out.reshape(*input_shape, -1)
-        return o_proj(out)
+        return attn_module.o_proj(out)
 
     return patched_forward
 
