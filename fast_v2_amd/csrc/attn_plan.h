@@ -142,7 +142,9 @@ inline void plan_ring_chunk(const fdllm_kv_attn_desc* d, int R, int64_t max_len,
 // Split-KV decode: by default the kernel partitions the keys itself from the device-side
 // lengths over S slots per KV head (S * Hkv ~ one workgroup per CU); a caller-given
 // kv_split fixes the keys per split instead.
-inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl) {
+// lean: without the slots and key ranges that only speed needs, for a caller whose workspace
+// is of the size such a plan takes.
+inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl, bool lean = false) {
   FDLLM_CHECK_ARG(d != nullptr, "fdllm_kv_attn: null descriptor");
   pl->ws_unit_off = 0;
   pl->ring = false;
@@ -268,7 +270,7 @@ inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl) {
         const int64_t round = (kDecodeSlotsTarget + hkv - 1) / hkv;
         slots = std::max<int64_t>(round, (B * min_splits + round - 1) / round * round);
         // (what the library's scratch holds without the rounding keeps fitting it)
-        if (slots * hkv * 64 * (d->head_dim + 2) * 4 > kScratchSlotBytes) slots = std::max(round, B * min_splits);
+        if (lean || slots * hkv * 64 * (d->head_dim + 2) * 4 > kScratchSlotBytes) slots = std::max(round, B * min_splits);
         pl->n_splits = static_cast<int>(slots);
         split_possible = slots > B;
       } else {
@@ -377,8 +379,8 @@ inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl) {
                           d->k_stride_slot >= 128 && d->v_stride_slot >= 128 && d->k_stride_slot < (1 << 24) &&
                           d->v_stride_slot < (1 << 24) && (pl->R + 255) / 256 < 65536 &&
                           (d->k_new == nullptr || d->new_stride_s >= 128);
-  int64_t ring_splits = 1, ring_tiles = 1;
-  if (ring_shape) plan_ring_chunk(d, pl->R, max_len, &ring_splits, &ring_tiles);
+  int64_t ring_splits = 1, ring_tiles = std::max<int64_t>(1, (max_len + kKT - 1) / kKT);
+  if (ring_shape && !lean) plan_ring_chunk(d, pl->R, max_len, &ring_splits, &ring_tiles);
   pl->ring = ring_shape && (ring_splits > 1 || !prefill_shape);
   if (prefill_shape && !pl->ring) {
     pl->kind = kPlanPrefill;

@@ -3960,6 +3960,10 @@ extern "C" int fdllm_kv_attn_fwd(const fdllm_kv_attn_desc* d, void* workspace, s
   Plan pl;
   const int rc = make_plan(d, &pl);
   if (rc != FDLLM_OK) return rc;
+  Plan lean;
+  if (workspace_bytes < plan_workspace_bytes(d, pl) && make_plan(d, &lean, true) == FDLLM_OK &&
+      workspace_bytes >= plan_workspace_bytes(d, lean))
+    pl = lean;
   return kv_attn_launch(d, pl, workspace, workspace_bytes, stream);
 }
 

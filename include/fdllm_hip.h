@@ -239,7 +239,9 @@ typedef struct fdllm_kv_attn_desc {
  * workspaces. */
 int fdllm_kv_attn_workspace_size(const fdllm_kv_attn_desc* desc, size_t* bytes);
 
-/* Launch the attention described by `desc` on `stream`. */
+/* Launch the attention described by `desc` on `stream`. A smaller workspace (none, where
+ * that is enough) that fits the call without the key splits that only speed asks for is
+ * accepted too; the call then runs without them. */
 int fdllm_kv_attn_fwd(const fdllm_kv_attn_desc* desc, void* workspace, size_t workspace_bytes,
                       void* stream);
 

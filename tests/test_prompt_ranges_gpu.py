@@ -1,5 +1,6 @@
 """Prompts of few row blocks: the ring prefill kernel with and without key ranges against
 float64 and against the general kernel (decode_kernel=False) over the forms it takes."""
+import ctypes
 import itertools
 
 import pytest
@@ -109,3 +110,35 @@ def test_prompt_graph_replay(gpu):
             graph.replay()
             assert torch.equal(out, ops.block_attn(q, k, v, seqlens, mask_mode=_ffi.MASK_CAUSAL))
             s.synchronize()
+
+
+def _c_call(q, k, v, seqlens, mode, ws_bytes):
+    out = torch.empty_like(q)
+    d = ops._attn_desc(q, k, v, seqlens, out, D ** -0.5, mode, 32, None, None, 0, 0)
+    need = ctypes.c_size_t(0)
+    _ffi.check(_ffi.lib().fdllm_kv_attn_workspace_size(ctypes.byref(d), ctypes.byref(need)), "size")
+    assert need.value > ws_bytes
+    ws = torch.zeros(max(ws_bytes, 16), dtype=torch.uint8, device="cuda")
+    rc = _ffi.lib().fdllm_kv_attn_fwd(ctypes.byref(d), ws.data_ptr() if ws_bytes else None, ws_bytes,
+                                      _ffi.stream_ptr(q.device))
+    torch.cuda.synchronize()
+    return rc, out
+
+
+def test_workspace_of_a_plan_without_ranges(gpu):
+    """A prompt without a workspace runs whole; a decode call with the slots it cannot do
+    without runs on those; less is refused."""
+    q, k, v, _, _, _ = _case(1, 500, (28, 4), 1203, "contiguous", torch.bfloat16, 3)
+    lens = torch.tensor([1203], dtype=torch.int32, device="cuda")
+    rc, out = _c_call(q, k, v, lens, _ffi.MASK_CAUSAL, 0)
+    assert rc == _ffi.FDLLM_OK
+    torch.testing.assert_close(out.double(), _ref(q, k, v, None, [1203], [703], _ffi.MASK_CAUSAL), atol=1e-2, rtol=1e-2)
+
+    q, k, v, _, _, _ = _case(33, 2, (8, 4), 5152, "contiguous", torch.bfloat16, 4)  # two splits each: 66 slots, or 128
+    lens = torch.tensor([40 * i + 5 for i in range(33)], dtype=torch.int32, device="cuda")
+    bytes_ = 64 * 1024 + 66 * 4 * 64 * 8 + 66 * 4 * 64 * 128 * 4
+    rc, out = _c_call(q, k, v, lens, _ffi.MASK_SEQLEN, bytes_)
+    assert rc == _ffi.FDLLM_OK
+    want = _ref(q, k, v, None, lens.tolist(), (lens - 2).tolist(), _ffi.MASK_SEQLEN)
+    torch.testing.assert_close(out.double(), want, atol=1e-2, rtol=1e-2)
+    assert _c_call(q, k, v, lens, _ffi.MASK_SEQLEN, bytes_ - 256)[0] == _ffi.FDLLM_ERR_WORKSPACE
