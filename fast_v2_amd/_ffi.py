@@ -219,3 +219,26 @@ def dtype_code(dt: torch.dtype) -> int:
 def stream_ptr(device: torch.device) -> int:
     """The current stream's handle (the raw lookup: a Stream object takes 1.2 us to make)."""
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
+HOST_PATH = Path(__file__).resolve().parent / "lib" / "fdllm_host.so"
+# in the order of csrc/host_calls.cpp's Api
+_HOST_APIS = ("fdllm_last_error", "fdllm_kv_attn_workspace_size", "fdllm_kv_attn_fwd", "fdllm_gather_rmsnorm",
+              "fdllm_scatter_rows", "fdllm_add_rmsnorm", "fdllm_qkv_rope_workspace_size",
+              "fdllm_qkv_rope_kv_write_ws", "fdllm_linear_workspace_size", "fdllm_linear",
+              "fdllm_unmask_workspace_size", "fdllm_unmask_step_ws")
+
+
+def host_calls(buffers: dict, get):
+    """The module of the calls' native host side (csrc/host_calls.cpp), bound to this
+    library and to a workspace dictionary and its ``get``."""
+    import importlib.util
+    if not HOST_PATH.exists():
+        raise RuntimeError(f"{HOST_PATH} is not built; run `python -m fast_v2_amd.build` first")
+    handle = lib()
+    spec = importlib.util.spec_from_file_location("fdllm_host", HOST_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    addr = tuple(ctypes.cast(getattr(handle, name), _c_vp).value for name in _HOST_APIS)
+    mod.init(addr, torch._C._cuda_getCurrentRawStream, buffers, get)
+    return mod

@@ -5,7 +5,7 @@
     python -m fast_v2_amd.build --timeline   # also the instrumented profiling build
 
 The libraries land in fast_v2_amd/lib/ so they travel with the source tree:
-libfdllm_hip.so (the operators), libfdllm_probes.so (the measurement probes bench.py
+libfdllm_hip.so (the operators), fdllm_host.so (their calls' host side), libfdllm_probes.so (the measurement probes bench.py
 times the calls against) and, on request, libfdllm_hip_timeline.so.
 """
 from __future__ import annotations
@@ -33,6 +33,10 @@ PROBES_HEADER = REPO_DIR / "include" / "fdllm_probes.h"
 SOURCES = [CSRC / "gather_rmsnorm.hip", CSRC / "block_attn.hip", CSRC / "rope_kv.hip", CSRC / "sampler.hip",
            CSRC / "linear.hip"]
 DEPS = SOURCES + [CSRC / "fdllm_common.h", CSRC / "skinny_gemm.h", CSRC / "attn_plan.h", CSRC / "host_errors.h", HEADER]
+# the calls' host side (a CPython module over torch's C++ API, no device code)
+HOST_LIB_PATH = LIB_DIR / "fdllm_host.so"
+HOST_SOURCES = [CSRC / "host_calls.cpp"]
+HOST_DEPS = HOST_SOURCES + [HEADER]
 PROBES_SOURCES = [CSRC / "probes.hip"]
 PROBES_DEPS = PROBES_SOURCES + [PROBES_HEADER]
 
@@ -63,6 +67,19 @@ def hipcc_path() -> str:
     raise RuntimeError("hipcc not found (looked at $HIPCC, PATH and /opt/rocm/bin/hipcc)")
 
 
+def _host_command(out: Path) -> list:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    return [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *[a for d in inc for a in ("-isystem", d)], *[str(x) for x in HOST_SOURCES],
+            *[a for d in cpp_extension.library_paths() for a in ("-L", d)],
+            "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-o", str(out)]
+
+
 def _stale(path: Path, deps) -> bool:
     if not path.exists():
         return True
@@ -73,7 +90,7 @@ def _stale(path: Path, deps) -> bool:
 def needs_build(timeline: bool = False) -> bool:
     """True if the operator or probe library (and, with ``timeline``, the instrumented
     build) is missing or older than one of its sources."""
-    return (_stale(LIB_PATH, DEPS) or _stale(PROBES_LIB_PATH, PROBES_DEPS)
+    return (_stale(LIB_PATH, DEPS) or _stale(PROBES_LIB_PATH, PROBES_DEPS) or _stale(HOST_LIB_PATH, HOST_DEPS)
             or (timeline and _stale(TIMELINE_LIB_PATH, DEPS)))
 
 
@@ -88,6 +105,11 @@ def build(force: bool = True, verbose: bool = False, timeline: bool = False) -> 
     if timeline:
         jobs.append((TIMELINE_LIB_PATH, ["-DFDLLM_TIMELINE=1"], SOURCES))
     procs = []
+    tmp = HOST_LIB_PATH.with_suffix(f".so.tmp{os.getpid()}")
+    cmd = _host_command(tmp)
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    procs.append((HOST_LIB_PATH, tmp, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)))
     for path, extra, sources in jobs:
         tmp = path.with_suffix(f".so.tmp{os.getpid()}")
         cmd = [hipcc_path(), *HIPCC_FLAGS, *extra, "-I", str(REPO_DIR / "include"),
@@ -103,7 +125,7 @@ def build(force: bool = True, verbose: bool = False, timeline: bool = False) -> 
         msgs = [l for l in (err or "").splitlines() if noise not in l]
         if proc.returncode != 0:
             tmp.unlink(missing_ok=True)
-            errors.append(f"hipcc failed for {path.name}:\n" + "\n".join(msgs))
+            errors.append(f"compiler failed for {path.name}:\n" + "\n".join(msgs))
             continue
         if verbose and msgs:
             print("\n".join(msgs), file=sys.stderr)

@@ -82,6 +82,20 @@ class _Workspace:
 
 
 _WORKSPACE = _Workspace()
+
+
+class _Host:
+    """The native host side of the calls (csrc/host_calls.cpp), loaded by the first call on a
+    GPU tensor. Its functions return None for a call that is not in the plain form."""
+
+    def __getattr__(self, name):
+        mod = _ffi.host_calls(_WORKSPACE._bufs, _WORKSPACE.get)
+        for fn in ("attn", "gather", "scatter", "add_norm", "linear", "linear_takes", "qkv", "unmask"):
+            setattr(self, fn, getattr(mod, fn))
+        return self.__dict__[name]
+
+
+_HOST = _Host()
 _COUNTER_BYTES = 64 * 1024  # arrival counters at the head of a workspace
 
 
@@ -104,6 +118,10 @@ def gather_rmsnorm(
     weight  [H] or None (then norm_mode must be NORM_PLAIN)
     Returns (normed [B, T, H], gathered [B, T, H] or None), both in hidden's dtype.
     """
+    if hidden.is_cuda:
+        done = _HOST.gather(hidden, indices, weight, eps, norm_mode, with_gathered)
+        if done is not None:
+            return done
     if hidden.dim() != 3 or indices.dim() != 2 or indices.shape[0] != hidden.shape[0]:
         raise RuntimeError(
             f"gather_rmsnorm: expected hidden [B,S,H] and indices [B,T]; got "
@@ -139,6 +157,10 @@ def add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: Optional[torch.
     """``s = x + residual`` (rounded to the rows' dtype) and the RMSNorm of ``s`` in one
     pass over the rows (modeling.py:465-488, 427-432). x, residual [..., H] bf16 / fp16 of
     one shape, H a multiple of 8 (at most 4096). Returns (s, normed), both new tensors."""
+    if x.is_cuda:
+        done = _HOST.add_norm(x, residual, weight, eps, norm_mode)
+        if done is not None:
+            return done
     if x.shape != residual.shape or x.dtype != residual.dtype:
         raise RuntimeError("add_rmsnorm: x and residual must share shape and dtype")
     dev = _require_gpu(x, residual, *([weight] if weight is not None else []))
@@ -188,6 +210,8 @@ def scatter_rows(values: torch.Tensor, indices: torch.Tensor,
     unspecified, and may differ between the two destinations).
 
     Returns ``current`` (None when it is not given)."""
+    if values.is_cuda and _HOST.scatter(values, indices, cache, current):
+        return current
     dests = [cache] + ([current] if current is not None else [])
     if values.dim() != 3 or indices.dim() != 2 or any(d.dim() != 3 for d in dests):
         raise RuntimeError("scatter_rows: expected values/cache/current [B,*,H] and indices [B,T]")
@@ -298,6 +322,15 @@ def block_attn(
     workgroups (runs that cross sequence boundaries) instead of splitting each sequence
     on its own.
     """
+    flags = ((0 if decode_kernel else _ffi.ATTN_NO_DECODE_KERNEL)
+             | (_ffi.ATTN_ALL_HEADS_DECODE if all_heads_decode else 0)
+             | (_ffi.ATTN_CACHE_WRITE_KERNEL if cache_write_kernel else 0)
+             | (_ffi.ATTN_BALANCED_SPLITS if balanced_splits else 0))
+    if out is None and kv_split == 0 and q.is_cuda:
+        done = _HOST.attn(q, k_cache, v_cache, cache_seqlens, softmax_scale, mask_mode, mask_block, q_start,
+                          page_table, page_size, k_new, v_new, flags)
+        if done is not None:
+            return done
     if q.dim() != 4 or k_cache.dim() != 4 or v_cache.dim() != 4:
         raise RuntimeError("block_attn: q, k_cache and v_cache must be 4-D (BSHD)")
     tensors = [q, k_cache, v_cache, cache_seqlens]
@@ -351,11 +384,7 @@ def block_attn(
     if softmax_scale is None:
         softmax_scale = D ** -0.5
     desc = _attn_desc(q, k_cache, v_cache, cache_seqlens, out, softmax_scale, mask_mode,
-                      mask_block, q_start, page_table, page_size, kv_split,
-                      (0 if decode_kernel else _ffi.ATTN_NO_DECODE_KERNEL)
-                      | (_ffi.ATTN_ALL_HEADS_DECODE if all_heads_decode else 0)
-                      | (_ffi.ATTN_CACHE_WRITE_KERNEL if cache_write_kernel else 0)
-                      | (_ffi.ATTN_BALANCED_SPLITS if balanced_splits else 0), k_new, v_new)
+                      mask_block, q_start, page_table, page_size, kv_split, flags, k_new, v_new)
     L = _ffi.lib()
     need = ctypes.c_size_t(0)
     _ffi.check(L.fdllm_kv_attn_workspace_size(ctypes.byref(desc), ctypes.byref(need)),
@@ -555,6 +584,11 @@ def qkv_rope_kv_write(
     (utils/attention_backends.py:837-842). The projections sum in fp32 and round once
     after the bias, as a 16-bit linear layer does, in a different order than a library
     GEMM. head_dim 128, hidden a multiple of 64."""
+    if x.is_cuda and q_out is None and not kv_out:
+        done = _HOST.qkv(x, wq, bq, wk, bk, wv, bv, cos, sin, k_cache, v_cache, write_start, write_offset, k_block,
+                         v_block, block_offset, head_dim)
+        if done is not None:
+            return done
     d, dims, keep = _qkv_desc(x, wq, bq, wk, bk, wv, bv, head_dim)
     B, S, Hq, Hkv, D, dev = dims
     q_out, kv_o, kept = _rope_dest_desc(d.rope, B, S, Hq, Hkv, D, x.dtype, dev, cos, sin, k_cache, v_cache,
@@ -593,6 +627,8 @@ def linear_fits(x: torch.Tensor, *weights: torch.Tensor, bias: Optional[torch.Te
     Below 128 rows a layer is bound by reading its weights once; above, by the products,
     where the library's tiles are the better ones."""
     w = weights[0]
+    if len(weights) == 1 and x.is_cuda and _HOST.linear_takes(x, w, bias):
+        return True
     if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or x.dim() < 2 or w.dim() != 2:
         return False
     n, k = w.shape
@@ -635,9 +671,24 @@ def _linear(x, w, w_up, bias):
     return out
 
 
+def try_linear(x: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tensor] = None,
+               bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``linear`` (``gated_linear`` with ``up_weight``) where ``linear_fits`` holds, else None."""
+    done = _HOST.linear(x, weight, up_weight, bias)
+    if done is None:
+        ws = (weight,) if up_weight is None else (weight, up_weight)
+        if linear_fits(x, *ws, bias=bias):
+            return _linear(x, weight, up_weight, bias)
+    return done
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x @ weight.T + bias`` of at most 128 rows (F.linear's shapes), summed in fp32 and
     rounded once; the weights are streamed once (``linear_fits`` states what it takes)."""
+    if x.is_cuda:
+        done = _HOST.linear(x, weight, None, bias)
+        if done is not None:
+            return done
     if not linear_fits(x, weight, bias=bias):
         raise RuntimeError(f"linear: unsupported layer (x {tuple(x.shape)} {x.dtype} on {x.device}, weight "
                            f"{tuple(weight.shape)} {weight.dtype})")
@@ -647,6 +698,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
 def gated_linear(x: torch.Tensor, gate_weight: torch.Tensor, up_weight: torch.Tensor) -> torch.Tensor:
     """``silu(x @ gate_weight.T) * (x @ up_weight.T)`` of at most 128 rows in one kernel,
     rounded where the two layers and ``silu_mul`` round (modeling.py:164)."""
+    if x.is_cuda:
+        done = _HOST.linear(x, gate_weight, up_weight, None)
+        if done is not None:
+            return done
     if not linear_fits(x, gate_weight, up_weight):
         raise RuntimeError(f"gated_linear: unsupported layers (x {tuple(x.shape)} {x.dtype} on {x.device}, weights "
                            f"{tuple(gate_weight.shape)} {gate_weight.dtype})")
@@ -690,6 +745,9 @@ def unmask_step(logits: torch.Tensor, tokens: torch.Tensor, mask_id: int, thresh
         raise RuntimeError("unmask_step: finished must be a contiguous bool / uint8 [B]")
     if scratch is None or scratch.row_tok.shape != (B, L) or scratch.row_tok.device != dev:
         scratch = UnmaskScratch(B, L, dev)
+    if _HOST.unmask(logits, tokens, mask_id, threshold, row_offset, shift, finished,
+                    -1 if stop_token is None else stop_token, scratch.row_tok, scratch.row_conf, scratch.counts):
+        return scratch
     need = ctypes.c_size_t(0)
     _ffi.check(_ffi.lib().fdllm_unmask_workspace_size(logits.shape[2], B, L, ctypes.byref(need)),
                "fdllm_unmask_workspace_size")
