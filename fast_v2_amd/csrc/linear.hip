@@ -1,4 +1,4 @@
-// Linear layers of a few token rows (fdllm_linear): the o_proj, MLP and lm_head products
+// Linear layers of a few token rows (fdllm_linear), such as the MLP and lm_head products
 // of a diffusion step, on the weight-streaming kernel of skinny_gemm.h, plain (with an
 // optional bias) or with the MLP's gate and up projections in one pass and their
 // SiLU-gated product as the epilogue (modeling.py:153-166).

@@ -422,7 +422,7 @@ int fdllm_qkv_rope_kv_write_ws(const fdllm_qkv_rope_desc* desc, void* workspace,
  * Without one (NULL) the weight rows are not cut over more workgroups than there are
  * 64-row tiles: slower where out_features is small.
  *
- * Replaces: o_proj, gate_proj / up_proj / act_fn, down_proj and lm_head of the model
+ * Replaces: gate_proj / up_proj / act_fn, down_proj and lm_head of the model
  * snapshot at the rows of a sub-block step (modeling.py:153-166, :325).
  * ------------------------------------------------------------------------- */
 int fdllm_linear_workspace_size(int rows, int out_features, int in_features, int gated, size_t* bytes);
