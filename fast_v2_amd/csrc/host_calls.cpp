@@ -48,7 +48,6 @@ constexpr int kApis = 12;
 PyObject* g_stream = nullptr;   // torch's raw stream lookup: device index -> handle
 PyObject* g_buffers = nullptr;  // ops._Workspace's dictionary: (device index, stream) -> tensor
 PyObject* g_get = nullptr;      // ops._Workspace.get
-constexpr int64_t kCounterBytes = 64 * 1024;
 
 // Raised inside a call for "not the plain form".
 struct NotPlain {};
@@ -461,10 +460,10 @@ PyObject* qkv(PyObject* const* a, Py_ssize_t n) {
 }
 
 // logits, tokens, mask_id, threshold, row_offset, shift, finished | None, stop (-1: none),
-// row_tok, row_conf, counts -> True
+// row_tok, row_conf, counts, parts -> True
 PyObject* unmask(PyObject* const* a, Py_ssize_t n) {
-  arity(n, 11);
-  const Tensor &lg = tensor(a[0]), &tok = tensor(a[1]), &rt = tensor(a[8]), &rc = tensor(a[9]), &cn = tensor(a[10]);
+  arity(n, 12);
+  const Tensor &lg = tensor(a[0]), &tok = tensor(a[1]), &rt = tensor(a[8]), &rc = tensor(a[9]), &cn = tensor(a[10]), &parts = tensor(a[11]);
   const Opt fin(a[6]);
   plain(lg.dim() == 3 && tok.dim() == 2 && tok.size(0) == lg.size(0) && tok.device() == lg.device() &&
         half_type(lg.scalar_type()) && lg.stride(2) == 1 && tok.scalar_type() == at::kLong && tok.stride(1) == 1);
@@ -477,17 +476,16 @@ PyObject* unmask(PyObject* const* a, Py_ssize_t n) {
   const long offset = integer(a[4]), shift = integer(a[5]), mask = integer(a[2]), stop = integer(a[7]);
   const float threshold = static_cast<float>(number(a[3]));
   plain(offset >= INT32_MIN && offset <= INT32_MAX && shift >= INT32_MIN && shift <= INT32_MAX);
-  size_t need = 0, have = 0;
+  size_t need = 0;
   check(api.unmask_size(static_cast<int>(V), static_cast<int>(B), static_cast<int>(L), &need), "fdllm_unmask_workspace_size");
+  plain(parts.device() == lg.device() && parts.scalar_type() == at::kByte && static_cast<size_t>(parts.numel()) >= need);
   const Stream s(lg);
-  // past the arrival counters that other calls keep at the head of the stream's scratch
-  char* ws = static_cast<char*>(s.workspace(kCounterBytes + need, lg, &have));
   check(launch([&] { return api.unmask(lg.data_ptr(), lg.stride(0), lg.stride(1), static_cast<int>(V), static_cast<int>(offset),
                    static_cast<int>(shift), static_cast<int64_t*>(tok.data_ptr()), tok.stride(0),
                    static_cast<uint8_t*>(fin.ptr()), mask, threshold, stop,
                    static_cast<int64_t*>(rt.data_ptr()), static_cast<float*>(rc.data_ptr()),
                    static_cast<int32_t*>(cn.data_ptr()), static_cast<int>(B), static_cast<int>(L),
-                   dtype_code(lg.scalar_type()), ws + kCounterBytes, need, s.ptr); }),
+                   dtype_code(lg.scalar_type()), parts.data_ptr(), need, s.ptr); }),
         "fdllm_unmask_step_ws");
   Py_RETURN_TRUE;
 }

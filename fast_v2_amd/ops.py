@@ -96,7 +96,6 @@ class _Host:
 
 
 _HOST = _Host()
-_COUNTER_BYTES = 64 * 1024  # arrival counters at the head of a workspace
 
 
 # ---------------------------------------------------------------------------
@@ -710,12 +709,28 @@ def gated_linear(x: torch.Tensor, gate_weight: torch.Tensor, up_weight: torch.Te
 
 class UnmaskScratch:
     """Device buffers of one sampler (greedy token and confidence per position, four
-    counters), allocated once per (batch, positions, device)."""
+    counters, and the partial results that a step's two kernels hand over), kept from call
+    to call. One sampler's steps run in order on one stream; another sampler, on the same
+    stream or not, has buffers of its own."""
 
     def __init__(self, batch: int, positions: int, device):
         self.row_tok = torch.empty((batch, positions), dtype=torch.int64, device=device)
         self.row_conf = torch.empty((batch, positions), dtype=torch.float32, device=device)
         self.counts = torch.zeros(4, dtype=torch.int32, device=device)
+        self._parts: list = []  # the last one is in use; a captured step may hold an earlier one
+
+    def parts(self, nbytes: int) -> torch.Tensor:
+        if not self._parts or self._parts[-1].numel() < nbytes:
+            self._parts.append(torch.empty(nbytes, dtype=torch.uint8, device=self.counts.device))
+        return self._parts[-1]
+
+
+@functools.lru_cache(maxsize=1024)
+def _unmask_bytes(vocab: int, batch: int, positions: int) -> int:
+    need = ctypes.c_size_t(0)
+    _ffi.check(_ffi.lib().fdllm_unmask_workspace_size(vocab, batch, positions, ctypes.byref(need)),
+               "fdllm_unmask_workspace_size")
+    return need.value
 
 
 def unmask_step(logits: torch.Tensor, tokens: torch.Tensor, mask_id: int, threshold: float,
@@ -745,20 +760,19 @@ def unmask_step(logits: torch.Tensor, tokens: torch.Tensor, mask_id: int, thresh
         raise RuntimeError("unmask_step: finished must be a contiguous bool / uint8 [B]")
     if scratch is None or scratch.row_tok.shape != (B, L) or scratch.row_tok.device != dev:
         scratch = UnmaskScratch(B, L, dev)
+    # the two kernels' partials: the step's own memory, as another thread's step on this
+    # stream may be launched between them
+    need = _unmask_bytes(logits.shape[2], B, L)
+    parts = scratch.parts(need)
     if _HOST.unmask(logits, tokens, mask_id, threshold, row_offset, shift, finished,
-                    -1 if stop_token is None else stop_token, scratch.row_tok, scratch.row_conf, scratch.counts):
+                    -1 if stop_token is None else stop_token, scratch.row_tok, scratch.row_conf, scratch.counts, parts):
         return scratch
-    need = ctypes.c_size_t(0)
-    _ffi.check(_ffi.lib().fdllm_unmask_workspace_size(logits.shape[2], B, L, ctypes.byref(need)),
-               "fdllm_unmask_workspace_size")
-    # past the arrival counters that other calls keep at the head of the stream's scratch
-    ws = _WORKSPACE.get(_COUNTER_BYTES + need.value, dev)
     rc = _ffi.lib().fdllm_unmask_step_ws(
         logits.data_ptr(), logits.stride(0), logits.stride(1), logits.shape[2], int(row_offset), int(shift),
         tokens.data_ptr(), tokens.stride(0), _ptr(finished), int(mask_id), float(threshold),
         -1 if stop_token is None else int(stop_token),
         scratch.row_tok.data_ptr(), scratch.row_conf.data_ptr(), scratch.counts.data_ptr(),
-        B, L, _ffi.dtype_code(logits.dtype), ws.data_ptr() + _COUNTER_BYTES, need.value, _ffi.stream_ptr(dev))
+        B, L, _ffi.dtype_code(logits.dtype), parts.data_ptr(), need, _ffi.stream_ptr(dev))
     _ffi.check(rc, "fdllm_unmask_step_ws")
     return scratch
 

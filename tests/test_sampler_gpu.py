@@ -8,6 +8,8 @@ than torch's). The logits are drawn so that no confidence lies within an ulp of 
 threshold and no two probabilities tie after rounding except where planted (an
 exact tie between two equal logits, resolved to the first index).
 """
+import threading
+
 import pytest
 import torch
 
@@ -98,3 +100,44 @@ def test_unmask_chunk_edges(gpu, V, dtype, scale):
     best = top[..., 0].argmax(dim=-1)
     assert x.cpu().gather(1, best[:, None])[:, 0].tolist() == tok.gather(1, best[:, None])[:, 0].tolist()
     assert sc.counts.tolist()[:2] == [B, B * (L - 1)]
+
+
+def test_a_step_keeps_its_partials_to_itself(gpu):
+    """A step is two kernels, and another thread's step may be launched between them on the
+    same stream: what they hand over lies in the caller's scratch, not in the memory that a
+    stream's callers share."""
+    s = torch.cuda.Stream()
+    raw = torch.randn(2, 4, 40000, device=gpu).bfloat16()
+    x = torch.full((2, 4), 39999, dtype=torch.int64, device=gpu)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        sc = ops.unmask_step(raw, x, 39999, 2.0)
+        again = ops.unmask_step(raw, x, 39999, 2.0, scratch=sc)
+        other = ops.unmask_step(raw, x, 39999, 2.0)
+    s.synchronize()
+    assert (gpu.index, s.cuda_stream) not in ops._WORKSPACE._bufs
+    assert again is sc and len(sc._parts) == 1 and sc._parts[0].data_ptr() != other._parts[0].data_ptr()
+
+
+def test_steps_of_two_threads_on_one_stream(gpu):
+    g = torch.Generator().manual_seed(8)
+    B, L, V, steps = 2, 4, 33000, 300
+    raws = [(torch.randn(B, L, V, generator=g) * 3).bfloat16().to(gpu) for _ in range(2)]
+    want = [ops.unmask_step(r, torch.full((B, L), V, dtype=torch.int64, device=gpu), V, 2.0).row_tok for r in raws]
+    bad, gate = [0, 0], threading.Barrier(2)
+
+    def run(i):
+        x = torch.full((B, L), V, dtype=torch.int64, device=gpu)
+        sc = ops.UnmaskScratch(B, L, gpu)
+        toks = []
+        gate.wait()
+        for _ in range(steps):
+            x.fill_(V)
+            toks.append(ops.unmask_step(raws[i], x, V, 2.0, scratch=sc).row_tok.clone())
+        bad[i] = sum(not torch.equal(t, want[i]) for t in toks)
+
+    assert not torch.equal(want[0], want[1])
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert bad == [0, 0]
