@@ -171,20 +171,24 @@ __global__ __launch_bounds__(kThreads) void unmask_rows_kernel(const UnmaskArgs 
   __syncthreads();
   if (tid == 0) {
     for (int w = 1; w < kThreads / 64; ++w) cand = min(cand, si[w]);
+    if (cand >= a.V) cand = 0;  // no logit above -inf: argmax over NaN probabilities
     a.row_tok[b * a.L + i] = cand;
     a.row_conf[b * a.L + i] = pmax;
   }
 }
 
 // The unmask rule of one sequence on one wave: lane i < L is position i of the sub-block,
-// c its confidence and tok its token.
+// conf its confidence and tok its token. A position without a confidence (NaN: non-finite
+// logits) stays masked, so that the caller sees a step without progress and no token that
+// nothing backs.
 __device__ __forceinline__ void select_positions(const UnmaskArgs& a, int b, int i, float conf, int64_t tok) {
   const bool live = i < a.L;
   const bool fin = a.finished != nullptr && a.finished[b] != 0;
   int64_t* tp = a.tokens + b * a.tok_sb + i;
   const int64_t t = live ? *tp : 0;
   const bool masked = live && t == a.mask_id && !fin;
-  const float c = masked ? conf : -INFINITY;
+  const bool known = masked && conf == conf;
+  const float c = known ? conf : -INFINITY;
   bool unmask = c > a.threshold;
   // most confident masked position, first on ties (torch.argmax over the row)
   float cm = live ? c : -INFINITY;
@@ -199,7 +203,7 @@ __device__ __forceinline__ void select_positions(const UnmaskArgs& a, int b, int
     }
   }
   if (i == im) unmask = true;
-  unmask = unmask && masked;
+  unmask = unmask && known;
   if (unmask) *tp = tok;
   const bool stop_hit = unmask && a.stop_token >= 0 && tok == a.stop_token;
   const uint64_t stops = __builtin_amdgcn_ballot_w64(stop_hit);
@@ -345,7 +349,7 @@ __global__ __launch_bounds__(kChunkThreads) void unmask_chunks_kernel(const Unma
     }
     int nr = 0;
     for (int u = 0; u < NW; ++u) nr |= sn[u];
-    // a chunk of -inf has no index of its own: only a row of -inf would use it
+    // a chunk of -inf has no index of its own
     a.parts[(static_cast<int64_t>(b) * a.L + i) * a.n_chunks + chunk] =
         make_float4(m, s, __int_as_float(m == -INFINITY ? 0x7fffffff : idx), __int_as_float(nr));
   }
@@ -405,6 +409,7 @@ __global__ __launch_bounds__(kFinishThreads) void unmask_finish_kernel(const Unm
     cand = min(cand, first);
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) cand = min(cand, __shfl_xor(cand, o, kWave));
+    if (cand >= a.V) cand = 0;  // no logit above -inf: argmax over NaN probabilities
     if (lane == 0) {
       s_conf[i] = pmax;
       s_tok[i] = cand;

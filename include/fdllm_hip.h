@@ -447,6 +447,9 @@ int fdllm_linear(const void* x, int64_t x_stride_row, const void* w, const void*
  *   finished, counts[2] = rows whose position 0 is still masked, counts[3] =
  *   finished rows (all after the step).
  *
+ * A position without a probability (NaN: non-finite logits) stays masked and takes no part
+ * in the maximum; its tok is an index below `vocab` all the same.
+ *
  * tokens is int64 with the positions of a row contiguous; finished is a byte per
  * row or NULL; stop_token < 0 disables the stop rule. row_tok / row_conf are
  * [batch, num_positions] outputs, counts an int32[4] output. Two kernels on
@@ -466,7 +469,8 @@ int fdllm_unmask_step(const void* logits, int64_t logits_stride_b, int64_t logit
  * workgroups and read once. The same outputs (row_conf may differ where a sum in another
  * order crosses a rounding boundary of the logits' type). `workspace`
  * (fdllm_unmask_workspace_size bytes, 16-byte aligned) needs no initialisation; calls that
- * may overlap in time need separate ones. */
+ * may overlap in time, or whose two kernels may alternate on one stream (launched by
+ * several threads), need separate ones. */
 int fdllm_unmask_workspace_size(int vocab, int batch, int num_positions, size_t* bytes);
 int fdllm_unmask_step_ws(const void* logits, int64_t logits_stride_b, int64_t logits_stride_row, int vocab,
                          int row_offset, int shift, int64_t* tokens, int64_t tokens_stride_b,

@@ -13,7 +13,7 @@ import threading
 import pytest
 import torch
 
-from fast_v2_amd import ops
+from fast_v2_amd import _ffi, ops
 from fast_v2_amd.e2e import model as em
 from fast_v2_amd.e2e import sampler as es
 
@@ -141,3 +141,40 @@ def test_steps_of_two_threads_on_one_stream(gpu):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert bad == [0, 0]
+
+
+def _step_without_workspace(raw, x, mask_id, threshold):
+    """fdllm_unmask_step, the entry point that takes no workspace."""
+    sc = ops.UnmaskScratch(*x.shape, x.device)
+    _ffi.check(_ffi.lib().fdllm_unmask_step(
+        raw.data_ptr(), raw.stride(0), raw.stride(1), raw.shape[2], 0, 0, x.data_ptr(), x.stride(0), None, mask_id,
+        threshold, -1, sc.row_tok.data_ptr(), sc.row_conf.data_ptr(), sc.counts.data_ptr(), *x.shape,
+        _ffi.dtype_code(raw.dtype), _ffi.stream_ptr(x.device)), "fdllm_unmask_step")
+    return sc
+
+
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("V", [1000, 9001])
+def test_rows_without_a_finite_probability(gpu, V, workspace):
+    """Rows of -inf, of NaN and with one NaN or +inf among finite logits: the token lies in
+    the vocabulary (0 where nothing is above -inf, as argmax over NaN), the position stays
+    masked, and the others of its sequence follow the rule."""
+    B, L = 3, 4
+    raw = torch.randn(B, L, V, generator=torch.Generator().manual_seed(V)).bfloat16()
+    raw[0, 1] = float("-inf")
+    raw[0, 2] = float("nan")
+    raw[1] = float("nan")
+    raw[1, 3] = float("-inf")
+    raw[2, 0, 7] = float("inf")
+    raw[2, 1, 9] = float("nan") if workspace else float("inf")
+    x = torch.full((B, L), V, dtype=torch.int64, device=gpu)
+    rawg = raw.to(gpu)
+    print(f"case non-finite rows V={V} workspace={workspace}", flush=True)
+    sc = ops.unmask_step(rawg, x, V, 0.0, shift=0) if workspace else _step_without_workspace(rawg, x, V, 0.0)
+    bad = torch.tensor([[0, 1, 1, 0], [1, 1, 1, 1], [1, 1, 0, 0]], dtype=torch.bool, device=gpu)
+    assert torch.equal(sc.row_conf.isnan(), bad)
+    assert bool(((sc.row_tok >= 0) & (sc.row_tok < V)).all())
+    assert sc.row_tok[0, 1:3].tolist() == [0, 0] and sc.row_tok[1].tolist() == [0] * 4
+    # threshold 0: every position with a probability is unmasked
+    assert torch.equal(x == V, bad) and torch.equal(x[~bad], rawg.argmax(dim=-1)[~bad])
+    assert sc.counts.tolist() == [4, 8, 2, 0]
