@@ -312,13 +312,20 @@ __global__ __launch_bounds__(kChunkThreads) void unmask_chunks_kernel(const Unma
 #pragma unroll
   for (int u = 0; u < NW; ++u) m = fmaxf(m, sm[u]);
   // exp relative to the chunk's maximum (0 for a chunk of -inf: its sum is then zero; a NaN
-  // or +inf logit makes it NaN, as in a softmax)
+  // or +inf logit makes it NaN, as in a softmax), as exp2 of the product with log2 e in two
+  // parts: with one, the constant's rounding biases every term the same way. Error of a row's
+  // sum against 64 bits, rms over 128 rows of 152064 bf16 logits of N(0, 2): 4.5e-8, 6.9e-8
+  // with one part, 4.4e-8 with expf (which takes 4 us more), 7.1e-8 in unmask_rows_kernel;
+  // with one clear token per row 1.4e-7, 1.5e-7, 1.4e-7 and 6.5e-7.
   const float ref = m == -INFINITY ? 0.f : m;
   float s = 0.f;
 #pragma unroll
   for (int k = 0; k < kChunkVecs; ++k)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s += __builtin_amdgcn_exp2f((x[k][j] - ref) * 1.4426950408889634f);
+    for (int j = 0; j < 8; ++j) {
+      const float t = x[k][j] - ref;
+      s += __builtin_amdgcn_exp2f(__builtin_fmaf(t, 1.44269502f, t * 1.92596299e-8f));
+    }
   int idx = 0x7fffffff;
 #pragma unroll
   for (int k = kChunkVecs - 1; k >= 0; --k)
