@@ -119,6 +119,13 @@ struct Ref {  // owned reference
   Ref(const Ref&) = delete;
 };
 
+// A call's workspace, held until its kernels are launched.
+struct Workspace {
+  Tensor buf;
+  void* ptr = nullptr;
+  size_t bytes = 0;
+};
+
 // The current stream of a device, and its workspace.
 struct Stream {
   Ref index, handle;
@@ -126,22 +133,24 @@ struct Stream {
   explicit Stream(const Tensor& t)
       : index(PyLong_FromLong(t.device().index())), handle(PyObject_CallOneArg(g_stream, index.o)),
         ptr(PyLong_AsVoidPtr(handle.o)) {}
-  // at least `bytes`; the buffer stays alive in the dictionary (or its retired list)
-  void* workspace(size_t bytes, const Tensor& t, size_t* have) const {
+  // at least `bytes` (nothing for 0)
+  Workspace workspace(size_t bytes, const Tensor& t) const {
+    Workspace w;
+    if (bytes == 0) return w;
     Ref key(PyTuple_Pack(2, index.o, handle.o));
-    PyObject* buf = PyDict_GetItemWithError(g_buffers, key.o);
-    if (!buf && PyErr_Occurred()) throw PyFailed{};
-    if (buf && static_cast<size_t>(THPVariable_Unpack(buf).numel()) >= bytes) {
-      const Tensor& w = THPVariable_Unpack(buf);
-      *have = w.numel();
-      return w.data_ptr();
+    PyObject* have = PyDict_GetItemWithError(g_buffers, key.o);
+    if (!have && PyErr_Occurred()) throw PyFailed{};
+    if (have && static_cast<size_t>(THPVariable_Unpack(have).numel()) >= bytes) {
+      w.buf = THPVariable_Unpack(have);
+    } else {
+      Ref dev(THPDevice_New(t.device()));
+      Ref size(PyLong_FromSize_t(bytes));
+      Ref made(PyObject_CallFunctionObjArgs(g_get, size.o, dev.o, nullptr));
+      w.buf = THPVariable_Unpack(made.o);
     }
-    Ref dev(THPDevice_New(t.device()));
-    Ref size(PyLong_FromSize_t(bytes));
-    Ref made(PyObject_CallFunctionObjArgs(g_get, size.o, dev.o, nullptr));
-    const Tensor& w = THPVariable_Unpack(made.o);
-    *have = w.numel();
-    return w.data_ptr();
+    w.ptr = w.buf.data_ptr();
+    w.bytes = w.buf.numel();
+    return w;
   }
 };
 
@@ -249,11 +258,11 @@ PyObject* attn(PyObject* const* a, Py_ssize_t n) {
     d.v_new = vn.ptr();
     d.new_stride_b = kn->stride(0), d.new_stride_s = kn->stride(1), d.new_stride_h = kn->stride(2);
   }
-  size_t need = 0, have = 0;
+  size_t need = 0;
   check(api.attn_size(&d, &need), "fdllm_kv_attn_workspace_size");
   const Stream s(q);
-  void* ws = need ? s.workspace(need, q, &have) : nullptr;
-  check(launch([&] { return api.attn(&d, ws, have, s.ptr); }), "fdllm_kv_attn_fwd");
+  const Workspace ws = s.workspace(need, q);
+  check(launch([&] { return api.attn(&d, ws.ptr, ws.bytes, s.ptr); }), "fdllm_kv_attn_fwd");
   return wrap(std::move(out));
 }
 
@@ -372,12 +381,12 @@ PyObject* linear(PyObject* const* a, Py_ssize_t n) {
   auto sizes = x.sizes().vec();
   sizes.back() = N;
   Tensor out = empty(sizes, x);
-  size_t need = 0, have = 0;
+  size_t need = 0;
   check(api.linear_size(m, N, K, up ? 1 : 0, &need), "fdllm_linear_workspace_size");
   const Stream s(x);
-  void* ws = need ? s.workspace(need, x, &have) : nullptr;
+  const Workspace ws = s.workspace(need, x);
   check(launch([&] { return api.linear(x.data_ptr(), K, w.data_ptr(), up.ptr(), bias.ptr(), out.data_ptr(), m, N, K,
-                   dtype_code(x.scalar_type()), ws, have, s.ptr); }),
+                   dtype_code(x.scalar_type()), ws.ptr, ws.bytes, s.ptr); }),
         "fdllm_linear");
   return wrap(std::move(out));
 }
@@ -451,11 +460,11 @@ PyObject* qkv(PyObject* const* a, Py_ssize_t n) {
   r.batch = static_cast<int>(B), r.seq_len = static_cast<int>(S), r.num_q_heads = static_cast<int>(Hq);
   r.num_kv_heads = static_cast<int>(Hkv), r.head_dim = static_cast<int>(D);
   r.dtype = dtype_code(x.scalar_type());
-  size_t need = 0, have = 0;
+  size_t need = 0;
   if (B * S <= 128) check(api.qkv_size(&d, &need), "fdllm_qkv_rope_workspace_size");
   const Stream s(x);
-  void* ws = need ? s.workspace(need, x, &have) : nullptr;
-  check(launch([&] { return api.qkv(&d, ws, have, s.ptr); }), "fdllm_qkv_rope_kv_write");
+  const Workspace ws = s.workspace(need, x);
+  check(launch([&] { return api.qkv(&d, ws.ptr, ws.bytes, s.ptr); }), "fdllm_qkv_rope_kv_write");
   return wrap(std::move(out));
 }
 

@@ -25,6 +25,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import math
+import threading
 from typing import Optional, Tuple
 
 import torch
@@ -56,12 +57,13 @@ class _Workspace:
     The buffer is zero-filled when allocated: the split-KV decode kernel's
     arrival counters must start at zero, and every call leaves them at zero.
     Partials are written before they are read, so nothing else needs clearing;
-    calls on one stream run in order and may share the buffer.
+    kernels on one stream run in order and may share the buffer.
 
     A buffer that is outgrown is retired, never freed: a HIP graph captured
     earlier on the stream keeps its address and writes counters and partials
     there on every replay, so the memory must not return to the caching
-    allocator while the process may still replay such a graph. Each retired
+    allocator while the process may still replay such a graph; another thread
+    may also be about to launch a call on it. Each retired
     buffer keeps its counters at zero (every call leaves them so), so a replay
     after any number of larger calls still starts from a clean state.
     """
@@ -69,15 +71,19 @@ class _Workspace:
     def __init__(self) -> None:
         self._bufs: dict = {}
         self._retired: list = []
+        self._lock = threading.RLock()  # a collection inside may run a finalizer that calls
 
     def get(self, nbytes: int, device: torch.device) -> torch.Tensor:
         key = (device.index, _ffi.stream_ptr(device))
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < nbytes:
-            if buf is not None:
-                self._retired.append(buf)
-            buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-            self._bufs[key] = buf
+            with self._lock:  # allocating lets other threads run: each buffer made is kept
+                buf = self._bufs.get(key)
+                if buf is None or buf.numel() < nbytes:
+                    buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+                    if key in self._bufs:
+                        self._retired.append(self._bufs[key])
+                    self._bufs[key] = buf
         return buf
 
 

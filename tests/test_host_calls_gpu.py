@@ -2,6 +2,7 @@
 the same calls: equal results in the plain forms, and the Python function's own conversions
 and refusals everywhere else."""
 import contextlib
+import threading
 
 import pytest
 import torch
@@ -214,3 +215,28 @@ def test_transforms_take_the_python_path(gpu):
     with FakeTensorMode(allow_non_fake_inputs=True):
         seen.append(host.attn(x[0], k, k, lens, None, 0, 32, None, None, 0, None, None, 0))
     assert seen == [None, None]
+
+
+def test_streams_and_threads(gpu):
+    """Native calls whose workspaces grow on two threads, each on a stream of its own and
+    then both on one stream: every result is the one of a call made alone."""
+    sizes = [(1, 200), (2, 900), (3, 2000), (4, 4000)]
+    data = [(_rnd(1, b, 8, 14, 128), _rnd(2, b, n, 2, 128), _rnd(3, b, n, 2, 128),
+             torch.full((b,), n, dtype=torch.int32, device="cuda")) for b, n in sizes]
+    want = [ops.block_attn(*a) for a in data]
+    torch.cuda.synchronize()
+    for streams in ([torch.cuda.Stream(), torch.cuda.Stream()], [torch.cuda.Stream()] * 2):
+        print(f"case threads, {len(set(streams))} streams", flush=True)
+        bad, gate = [-1, -1], threading.Barrier(2)
+
+        def run(i):
+            with torch.cuda.stream(streams[i]):
+                gate.wait()
+                outs = [(j, ops.block_attn(*data[j])) for _ in range(20) for j in range(4)]
+                streams[i].synchronize()
+                bad[i] = sum(not torch.equal(o, want[j]) for j, o in outs)
+
+        threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+        [t.start() for t in threads]
+        [t.join() for t in threads]
+        assert bad == [0, 0]
