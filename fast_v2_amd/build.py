@@ -32,7 +32,7 @@ PROBES_HEADER = REPO_DIR / "include" / "fdllm_probes.h"
 
 SOURCES = [CSRC / "gather_rmsnorm.hip", CSRC / "block_attn.hip", CSRC / "rope_kv.hip", CSRC / "sampler.hip",
            CSRC / "linear.hip"]
-DEPS = SOURCES + [CSRC / "fdllm_common.h", CSRC / "skinny_gemm.h", CSRC / "attn_plan.h", CSRC / "host_errors.h", HEADER]
+DEPS = SOURCES + [CSRC / "fdllm_common.h", CSRC / "skinny_gemm.h", CSRC / "attn_plan.h", CSRC / "launch_turn.h", CSRC / "host_errors.h", HEADER]
 # the calls' host side (a CPython module over torch's C++ API, no device code)
 HOST_LIB_PATH = LIB_DIR / "fdllm_host.so"
 HOST_SOURCES = [CSRC / "host_calls.cpp"]

@@ -40,6 +40,7 @@
 
 #include "fdllm_common.h"
 #include "attn_plan.h"
+#include "launch_turn.h"
 
 namespace fdllm {
 namespace {
@@ -3746,6 +3747,7 @@ int kv_attn_launch(const fdllm_kv_attn_desc* d, const Plan& pl, void* workspace,
   }
   const bool f16 = d->dtype == FDLLM_DTYPE_F16;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const WorkspaceTurn turn(need > 0 ? workspace : nullptr);
   if (pl.kind == kPlanF32) {
     // 4 FDLLM_F32_ROWS_PER_WAVE rows of one (sequence, KV head) per workgroup
     const dim3 grid = to_dim3(ls.main_grid);

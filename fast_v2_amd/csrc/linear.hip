@@ -2,6 +2,7 @@
 // of a diffusion step, on the weight-streaming kernel of skinny_gemm.h, plain (with an
 // optional bias) or with the MLP's gate and up projections in one pass and their
 // SiLU-gated product as the epilogue (modeling.py:153-166).
+#include "launch_turn.h"
 #include "skinny_gemm.h"
 
 namespace fdllm {
@@ -166,6 +167,7 @@ extern "C" int fdllm_linear(const void* x, int64_t x_stride_row, const void* w, 
   const uint16_t* w1 = static_cast<const uint16_t*>(w_up);
   const uint16_t* bi = static_cast<const uint16_t*>(bias);
   uint16_t* o = static_cast<uint16_t*>(out);
+  const WorkspaceTurn turn(need > 0 ? workspace : nullptr);
   if (dtype == FDLLM_DTYPE_BF16) {
     if (w1) launch<false>(a, bn, GatedEpi<bf16_t>{w0, w1, o, out_features, in_features}, s);
     else launch<false>(a, bn, LinearEpi<bf16_t>{w0, bi, o, out_features, in_features}, s);

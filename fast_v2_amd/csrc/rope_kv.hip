@@ -7,6 +7,7 @@
 // destination. V rows are copied in 16-byte vectors. The arithmetic rounds to the
 // 16-bit type after each product and after the sum, exactly as the eager
 // expression q * cos + rotate_half(q) * sin (utils/attention_backends.py:777-788).
+#include "launch_turn.h"
 #include "skinny_gemm.h"
 
 namespace fdllm {
@@ -569,6 +570,7 @@ extern "C" int fdllm_qkv_rope_kv_write_ws(const fdllm_qkv_rope_desc* d, void* wo
     k.w_stride_b = d->hidden * 2;
     k.cnt = static_cast<int*>(workspace);
     k.part = static_cast<uint8_t*>(workspace) + kSkinnyCounterBytes;
+    const WorkspaceTurn turn(need > 0 ? workspace : nullptr);
     if (r.dtype == FDLLM_DTYPE_BF16) skinny_launch<false, kSkinnyBN>(k, QkvEpi<bf16_t>{*d}, s);
     else skinny_launch<true, kSkinnyBN>(k, QkvEpi<f16_t>{*d}, s);
     FDLLM_RETURN_LAUNCH_STATUS("fdllm_qkv_rope_kv_write");

@@ -57,7 +57,9 @@ class _Workspace:
     The buffer is zero-filled when allocated: the split-KV decode kernel's
     arrival counters must start at zero, and every call leaves them at zero.
     Partials are written before they are read, so nothing else needs clearing;
-    kernels on one stream run in order and may share the buffer.
+    kernels on one stream run in order and may share the buffer (the library launches
+    the kernels of one call without another call's on that buffer in between, whichever
+    threads make the calls).
 
     A buffer that is outgrown is retired, never freed: a HIP graph captured
     earlier on the stream keeps its address and writes counters and partials

@@ -236,7 +236,8 @@ typedef struct fdllm_kv_attn_desc {
  * allocated: every call leaves the counters at zero again and writes every
  * partial it reads, so one workspace then serves any sequence of calls of any
  * sizes. Calls that may overlap in time (different streams) need separate
- * workspaces. */
+ * workspaces; threads that launch on one stream may share one (a call's kernels are
+ * launched without another call's on that workspace in between). */
 int fdllm_kv_attn_workspace_size(const fdllm_kv_attn_desc* desc, size_t* bytes);
 
 /* Launch the attention described by `desc` on `stream`. A smaller workspace (none, where

@@ -2,6 +2,7 @@
 float64 and against the general kernel (decode_kernel=False) over the forms it takes."""
 import ctypes
 import itertools
+import threading
 
 import pytest
 import torch
@@ -142,3 +143,29 @@ def test_workspace_of_a_plan_without_ranges(gpu):
     want = _ref(q, k, v, None, lens.tolist(), (lens - 2).tolist(), _ffi.MASK_SEQLEN)
     torch.testing.assert_close(out.double(), want, atol=1e-2, rtol=1e-2)
     assert _c_call(q, k, v, lens, _ffi.MASK_SEQLEN, bytes_ - 256)[0] == _ffi.FDLLM_ERR_WORKSPACE
+
+
+def test_calls_of_two_threads_on_one_stream(gpu):
+    """Calls of two kernels (a prompt with key ranges, a whole-block decode) and of one from
+    two threads on one stream, which share that stream's workspace."""
+    def call(b, sq, n, seed, mode):
+        q, k, v, _, _, _ = _case(b, sq, (28, 4), n, "contiguous", torch.bfloat16, seed)
+        return q, k, v, torch.full((b,), n, dtype=torch.int32, device="cuda"), mode
+    calls = [call(1, 300, 2048, 1, _ffi.MASK_CAUSAL), call(4, 32, 1500, 2, _ffi.MASK_SEQLEN),
+             call(4, 8, 1500, 3, _ffi.MASK_SEQLEN)]
+    run = [lambda c=c: ops.block_attn(*c[:4], mask_mode=c[4]) for c in calls]
+    want = [f() for f in run]
+    torch.cuda.synchronize()
+    s, gate, bad = torch.cuda.Stream(), threading.Barrier(2), [-1, -1]
+
+    def thread(i):
+        with torch.cuda.stream(s):
+            gate.wait()
+            got = [(j, run[j]()) for n in range(60) for j in ((0, 1, 2), (1, 2, 0))[i]]
+            s.synchronize()
+            bad[i] = sum(not torch.equal(o, want[j]) for j, o in got)
+
+    threads = [threading.Thread(target=thread, args=(i,)) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert bad == [0, 0]
