@@ -9,6 +9,7 @@ point raises ``RuntimeError``.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import threading
 from pathlib import Path
@@ -108,6 +109,7 @@ class QkvRopeDesc(ctypes.Structure):
 SIGNATURES = {
     "fdllm_abi_version": (_c_int, []),
     "fdllm_last_error": (ctypes.c_char_p, []),
+    "fdllm_exchange_capture_mode": (_c_int, [ctypes.POINTER(_c_int)]),
     "fdllm_gather_rmsnorm": (_c_int, [
         _c_vp, _c_i64, _c_i64,          # hidden, batch stride, row stride
         _c_vp, _c_i64,                  # indices, batch stride
@@ -204,6 +206,18 @@ def check(rc: int, what: str) -> None:
     if rc != FDLLM_OK:
         msg = lib().fdllm_last_error().decode(errors="replace")
         raise RuntimeError(f"{what} failed (code {rc}): {msg}")
+
+
+@contextlib.contextmanager
+def relaxed_capture():
+    """The calling thread may allocate and wait for other streams inside, also while a
+    stream of its own is being captured."""
+    mode = _c_int(2)
+    check(lib().fdllm_exchange_capture_mode(ctypes.byref(mode)), "fdllm_exchange_capture_mode")
+    try:
+        yield
+    finally:
+        check(lib().fdllm_exchange_capture_mode(ctypes.byref(mode)), "fdllm_exchange_capture_mode")
 
 
 def dtype_code(dt: torch.dtype) -> int:

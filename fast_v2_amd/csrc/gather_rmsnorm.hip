@@ -597,6 +597,19 @@ int dtype_size(int dtype) {
 
 extern "C" int fdllm_abi_version(void) { return FDLLM_ABI_VERSION; }
 
+extern "C" int fdllm_exchange_capture_mode(int* mode) {
+  using namespace fdllm;
+  FDLLM_CHECK_ARG(mode != nullptr && *mode >= 0 && *mode <= 2, "fdllm_exchange_capture_mode: mode must be 0, 1 or 2");
+  hipStreamCaptureMode m = static_cast<hipStreamCaptureMode>(*mode);
+  const hipError_t e = hipThreadExchangeStreamCaptureMode(&m);
+  if (e != hipSuccess) {
+    set_last_error("fdllm_exchange_capture_mode: %s", hipGetErrorString(e));
+    return static_cast<int>(e);
+  }
+  *mode = static_cast<int>(m);
+  return FDLLM_OK;
+}
+
 extern "C" const char* fdllm_last_error(void) { return fdllm::g_last_error; }
 
 extern "C" int fdllm_gather_rmsnorm(const void* hidden, int64_t hidden_batch_stride, int64_t hidden_row_stride,

@@ -68,6 +68,10 @@ class _Workspace:
     may also be about to launch a call on it. Each retired
     buffer keeps its counters at zero (every call leaves them so), so a replay
     after any number of larger calls still starts from a clean state.
+
+    A buffer that is first needed inside a capture is made and cleared outside of it: as
+    part of the graph it would be cleared by replays only, and counters of that stream's
+    eager calls, or of another graph captured there, would be whatever the memory held.
     """
 
     def __init__(self) -> None:
@@ -82,11 +86,28 @@ class _Workspace:
             with self._lock:  # allocating lets other threads run: each buffer made is kept
                 buf = self._bufs.get(key)
                 if buf is None or buf.numel() < nbytes:
-                    buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+                    buf = self._make(max(nbytes, 1 << 20), device)
                     if key in self._bufs:
                         self._retired.append(self._bufs[key])
                     self._bufs[key] = buf
         return buf
+
+    @staticmethod
+    def _make(nbytes: int, device: torch.device) -> torch.Tensor:
+        if device.type != "cuda":
+            return torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        with torch.cuda.device(device):
+            if not torch.cuda.is_current_stream_capturing():
+                return torch.zeros(nbytes, dtype=torch.uint8, device=device)
+            with _ffi.relaxed_capture():
+                for _ in range(64):  # torch hands out 32 streams in turn, some may be part of the capture
+                    side = torch.cuda.Stream(device)
+                    with torch.cuda.stream(side):
+                        if not torch.cuda.is_current_stream_capturing():
+                            buf = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+                            side.synchronize()
+                            return buf
+        raise RuntimeError("no stream outside the running capture to clear a workspace on; make one call before it")
 
 
 _WORKSPACE = _Workspace()

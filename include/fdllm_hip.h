@@ -67,6 +67,13 @@ extern "C" {
 #define FDLLM_ABI_VERSION 2
 int fdllm_abi_version(void);
 
+/* hipThreadExchangeStreamCaptureMode for callers that do not bind HIP themselves: sets the
+ * calling thread's stream-capture mode to *mode (hipStreamCaptureMode: 0 global,
+ * 1 thread-local, 2 relaxed) and returns the previous one in *mode. In the relaxed mode a
+ * thread may allocate memory and wait for other streams while a stream of its own is being
+ * captured. */
+int fdllm_exchange_capture_mode(int* mode);
+
 /* Human-readable description of the calling thread's last failure ("" if none). */
 const char* fdllm_last_error(void);
 

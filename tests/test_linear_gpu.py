@@ -98,3 +98,42 @@ def test_qkv_linear_is_the_fused_kernels_projection(gpu, rows):
     q_rot, (k_rot, v_out) = ops.qkv_rope_kv_write(x, *args, cos, sin, kv_out=True)
     q2, (k2, v2) = ops.rope_kv_write(q, k, v, cos, sin, kv_out=True)
     assert torch.equal(q_rot, q2) and torch.equal(k_rot, k2) and torch.equal(v_out, v2) and torch.equal(v, v2)
+
+
+def test_first_calls_of_a_stream_under_capture(gpu):
+    """A capture may be the first use of a stream: the workspace is cleared at once, so eager
+    calls on that stream before the first replay, the replays and a second graph captured
+    there all find their counters at zero."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x, w = _ints(g, 24, 4096, dtype=torch.bfloat16), _ints(g, 200, 4096, dtype=torch.bfloat16)
+    big = _ints(g, 4096, 4096, dtype=torch.bfloat16)
+    q, k, v = (torch.randn(2, n, h, 128, generator=g, device="cuda").bfloat16() for n, h in ((8, 28), (900, 4), (900, 4)))
+    lens = torch.tensor([900, 500], dtype=torch.int32, device="cuda")
+    xp = torch.randn(2, 8, 512, generator=g, device="cuda").bfloat16()
+    wp = [(torch.randn(n, 512, generator=g, device="cuda") * 0.05).bfloat16() for n in (512, 128, 128)]
+    cs = torch.randn(1, 8, 128, generator=g, device="cuda").bfloat16()
+
+    def calls():
+        return [ops.block_attn(q, k, v, lens), ops.linear(x, w), ops.linear(x, big),
+                ops.qkv_rope_kv_write(xp, wp[0], None, wp[1], None, wp[2], None, cs, cs)]
+
+    want = calls()
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    while (gpu.index, s.cuda_stream) in ops._WORKSPACE._bufs:  # streams come out of a small pool
+        s = torch.cuda.Stream()
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    outs = []
+    for graph in graphs:
+        with torch.cuda.graph(graph, stream=s):
+            outs.append(calls())
+    with torch.cuda.stream(s):
+        print("case eager before the first replay", flush=True)
+        assert all(torch.equal(a, b) for a, b in zip(calls(), want))
+        for i in (1, 0, 1, 0, 0):  # the graph captured second is replayed first
+            print(f"case replay of graph {i}", flush=True)
+            [o.zero_() for o in outs[i]]
+            graphs[i].replay()
+            assert all(torch.equal(a, b) for a, b in zip(outs[i], want))
+            assert all(torch.equal(a, b) for a, b in zip(calls(), want))
+    s.synchronize()
