@@ -441,6 +441,29 @@ inline size_t plan_workspace_bytes(const fdllm_kv_attn_desc*, const Plan& pl) {
   return pl.ws_o_bytes > 0 ? kCounterBytes + align256(pl.ws_ml_bytes) + pl.ws_o_bytes : 0;
 }
 
+// The plan of a call with a workspace of the caller's: without the splits that only speed
+// asks for where the workspace holds no more.
+inline int make_plan_within(const fdllm_kv_attn_desc* d, const void* workspace, size_t bytes, Plan* pl) {
+  const int rc = make_plan(d, pl);
+  if (rc != FDLLM_OK) return rc;
+  const size_t usable = workspace != nullptr && aligned16(workspace) ? bytes : 0;
+  Plan lean;
+  if (usable < plan_workspace_bytes(d, *pl) && make_plan(d, &lean, true) == FDLLM_OK &&
+      usable >= plan_workspace_bytes(d, lean))
+    *pl = lean;
+  return FDLLM_OK;
+}
+
+// The plan of a call on the library's scratch, which all of a device's calls share and which
+// a first call may not resolve under capture: prompts that can do without it do.
+inline int make_plan_noalloc(const fdllm_kv_attn_desc* d, Plan* pl) {
+  const int rc = make_plan(d, pl);
+  if (rc != FDLLM_OK || !pl->ring || plan_workspace_bytes(d, *pl) == 0) return rc;
+  Plan lean;
+  if (make_plan(d, &lean, true) == FDLLM_OK && lean.kind == kPlanPrefill) *pl = lean;
+  return FDLLM_OK;
+}
+
 // The rows of k_new / v_new are stored from inside the prefill kernels (plan kinds
 // prefill and split prefill, and general on the ring kernel; no explicit q_start, no FDLLM_ATTN_CACHE_WRITE_KERNEL);
 // otherwise a copy kernel stores them ahead of the attention.

@@ -3960,12 +3960,8 @@ extern "C" int fdllm_kv_attn_fwd(const fdllm_kv_attn_desc* d, void* workspace, s
                                  void* stream) {
   using namespace fdllm;
   Plan pl;
-  const int rc = make_plan(d, &pl);
+  const int rc = make_plan_within(d, workspace, workspace_bytes, &pl);
   if (rc != FDLLM_OK) return rc;
-  Plan lean;
-  if (workspace_bytes < plan_workspace_bytes(d, pl) && make_plan(d, &lean, true) == FDLLM_OK &&
-      workspace_bytes >= plan_workspace_bytes(d, lean))
-    pl = lean;
   return kv_attn_launch(d, pl, workspace, workspace_bytes, stream);
 }
 
@@ -3983,7 +3979,7 @@ extern "C" int fdllm_timeline_attach(void* stamps) {
 extern "C" int fdllm_kv_attn_fwd_noalloc(const fdllm_kv_attn_desc* d, void* stream) {
   using namespace fdllm;
   Plan pl;
-  int rc = make_plan(d, &pl);
+  int rc = make_plan_noalloc(d, &pl);
   if (rc != FDLLM_OK) return rc;
   const size_t need = plan_workspace_bytes(d, pl);
   if (need > kScratchBytes) {

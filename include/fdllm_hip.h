@@ -259,7 +259,8 @@ int fdllm_kv_attn_fwd(const fdllm_kv_attn_desc* desc, void* workspace, size_t wo
 /* fdllm_kv_attn_fwd without a workspace argument and without any allocation: the
  * split partials and arrival counters live in a device array of
  * FDLLM_KV_ATTN_SCRATCH_BYTES that the library holds on every device it runs on
- * until the process ends. Same kernels, same results as fdllm_kv_attn_fwd.
+ * until the process ends. Same kernels, same results as fdllm_kv_attn_fwd (for prompts of
+ * 2048 and more query rows per KV head, as fdllm_kv_attn_fwd without a workspace).
  *
  * No counterpart in the reference: it is for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid
@@ -269,8 +270,9 @@ int fdllm_kv_attn_fwd(const fdllm_kv_attn_desc* desc, void* workspace, size_t wo
  *     the automatic split (kv_split 0), in the default build, the scratch holds any sub-block decode
  *     (<= 64 query rows per KV head) of up to 64 sequences of at most 5120 keys
  *     with <= 8 KV heads, and any full-block decode (<= 256 rows per KV head) of up
- *     to 64 sequences of at most 10240 keys with <= 4 KV heads; calls that need no
- *     workspace (prefill) always fit.
+ *     to 64 sequences of at most 10240 keys with <= 4 KV heads; prompts of 2048 and
+ *     more query rows per KV head run without key ranges here, need no scratch and so
+ *     always fit (pages of >= 32 keys).
  *   - The first call on a device resolves the scratch, clears its counters on
  *     `stream` and waits for that clear (so later calls from any stream or thread
  *     start after it); it must not be made under stream capture

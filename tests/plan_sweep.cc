@@ -277,6 +277,44 @@ static void check_validation(fdllm_kv_attn_desc d, const Plan& pl) {
         describe(d));
 }
 
+// The plans for a smaller workspace and for the library's scratch.
+static void check_other_plans(const fdllm_kv_attn_desc& d, const Plan& pl) {
+  alignas(16) static unsigned char ws[16];
+  const size_t need = plan_workspace_bytes(&d, pl);
+  Plan lean, other;
+  memset(&lean, 0xA5, sizeof(lean));
+  CHECK(make_plan(&d, &lean, true) == FDLLM_OK, "no lean plan: %s", describe(d));
+  check_plan(d, lean);
+  const size_t least = plan_workspace_bytes(&d, lean);
+  CHECK(least <= need, "lean plan needs %zu of %zu: %s", least, need, describe(d));
+  if (d.batch > 0 && d.q_len > 0) check_launches(d, lean);
+  if (pl.ring) {
+    CHECK(d.head_dim == 128 && pl.R > 256 && pl.MT == 4 && pl.rows_per_wg == 256 && d.kv_split == 0 &&
+              !(d.flags & FDLLM_ATTN_NO_DECODE_KERNEL),
+          "ring shape: %s", describe(d));
+    CHECK(d.k_stride_slot >= 128 && d.v_stride_slot >= 128 && d.k_stride_slot < (1 << 24) &&
+              d.v_stride_slot < (1 << 24) && (d.k_new == nullptr || d.new_stride_s >= 128),
+          "ring strides: %s", describe(d));
+    CHECK(d.page_table == nullptr || (d.page_size >= 32 && plan_max_keys(&d) <= 65152), "ring pages: %s", describe(d));
+    CHECK(need <= FDLLM_KV_ATTN_SCRATCH_BYTES, "ring workspace %zu: %s", need, describe(d));
+  }
+  // with the plan's workspace: the plan; with the lean one's, at any address where that is
+  // nothing: a plan that fits
+  CHECK(make_plan_within(&d, ws, need, &other) == FDLLM_OK && plan_workspace_bytes(&d, other) == need,
+        "own workspace: %s", describe(d));
+  CHECK(make_plan_within(&d, ws, least, &other) == FDLLM_OK && plan_workspace_bytes(&d, other) <= least,
+        "lean workspace: %s", describe(d));
+  if (least == 0) {
+    const void* bad[] = {nullptr, ws + 8};
+    for (const void* p : bad)
+      CHECK(make_plan_within(&d, p, SIZE_MAX / 2, &other) == FDLLM_OK && plan_workspace_bytes(&d, other) == 0,
+            "no usable workspace: %s", describe(d));
+  }
+  // prompts of at least 2048 rows never touch the library's scratch
+  CHECK(make_plan_noalloc(&d, &other) == FDLLM_OK && plan_workspace_bytes(&d, other) <= need, "noalloc: %s", describe(d));
+  if (lean.kind == kPlanPrefill) CHECK(plan_workspace_bytes(&d, other) == 0, "noalloc prompt: %s", describe(d));
+}
+
 int main() {
   alignas(16) static unsigned char dev[256];  // stand-in device pointers: checked, never read
   static const int32_t table_dummy[1] = {0};
@@ -366,6 +404,7 @@ int main() {
                   if (pl.kind < 0 || pl.kind > 6) continue;
                   ++kinds[pl.kind];
                   check_plan(d, pl);
+                  check_other_plans(d, pl);
                   if (d.batch > 0 && d.q_len > 0) {
                     check_launches(d, pl);
                     check_validation(d, pl);

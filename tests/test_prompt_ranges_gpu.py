@@ -169,3 +169,22 @@ def test_calls_of_two_threads_on_one_stream(gpu):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert bad == [0, 0]
+
+
+def test_prompt_on_the_librarys_scratch(gpu):
+    """fdllm_kv_attn_fwd_noalloc runs a prompt of 2048 rows and more as fdllm_kv_attn_fwd
+    does without a workspace; a workspace size without a workspace counts as none."""
+    q, k, v, _, _, _ = _case(1, 800, (12, 2), 832, "contiguous", torch.bfloat16, 12)
+    lens = torch.tensor([832], dtype=torch.int32, device="cuda")
+    outs = []
+    for form in ("noalloc", "none", "null"):
+        out = torch.empty_like(q)
+        d = ops._attn_desc(q, k, v, lens, out, D ** -0.5, _ffi.MASK_CAUSAL, 32, None, None, 0, 0)
+        st = _ffi.stream_ptr(q.device)
+        rc = _ffi.lib().fdllm_kv_attn_fwd_noalloc(ctypes.byref(d), st) if form == "noalloc" else \
+            _ffi.lib().fdllm_kv_attn_fwd(ctypes.byref(d), None, 0 if form == "none" else 1 << 30, st)
+        _ffi.check(rc, form)
+        outs.append(out)
+    want = _ref(q, k, v, None, [832], [32], _ffi.MASK_CAUSAL)
+    torch.testing.assert_close(outs[0].double(), want, atol=1e-2, rtol=1e-2)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
