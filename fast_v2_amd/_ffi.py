@@ -253,6 +253,8 @@ def host_calls(buffers: dict, get):
     spec = importlib.util.spec_from_file_location("fdllm_host", HOST_PATH)
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
+    if mod.torch_version != torch.__version__:
+        raise RuntimeError(f"{HOST_PATH} is built for torch {mod.torch_version}, this is {torch.__version__}")
     addr = tuple(ctypes.cast(getattr(handle, name), _c_vp).value for name in _HOST_APIS)
     mod.init(addr, torch._C._cuda_getCurrentRawStream, buffers, get)
     return mod

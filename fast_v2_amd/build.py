@@ -75,6 +75,7 @@ def _host_command(out: Path) -> list:
     inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
     return [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DFDLLM_TORCH_VERSION="{torch.__version__}"',
             *[a for d in inc for a in ("-isystem", d)], *[str(x) for x in HOST_SOURCES],
             *[a for d in cpp_extension.library_paths() for a in ("-L", d)],
             "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-o", str(out)]

@@ -533,4 +533,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "fdllm_host", nullptr, -1, methods,
 
 }  // namespace
 
-extern "C" PyObject* PyInit_fdllm_host() { return PyModule_Create(&module); }
+extern "C" PyObject* PyInit_fdllm_host() {
+  PyObject* m = PyModule_Create(&module);
+  // torch's C++ API has no stable layout: the loader compares
+  if (m && PyModule_AddStringConstant(m, "torch_version", FDLLM_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -24,6 +24,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import logging
 import math
 import threading
 from typing import Optional, Tuple
@@ -31,6 +32,8 @@ from typing import Optional, Tuple
 import torch
 
 from . import _ffi
+
+_LOG = logging.getLogger(__name__)
 
 # ---------------------------------------------------------------------------
 # helpers
@@ -115,13 +118,28 @@ _WORKSPACE = _Workspace()
 
 class _Host:
     """The native host side of the calls (csrc/host_calls.cpp), loaded by the first call on a
-    GPU tensor. Its functions return None for a call that is not in the plain form."""
+    GPU tensor. Its functions return None for a call that is not in the plain form. Where it
+    cannot be loaded (it is built against one torch, the kernels' library against none), every
+    call takes its Python form, after one log entry."""
+
+    _CALLS = ("attn", "gather", "scatter", "add_norm", "linear", "linear_takes", "qkv", "unmask")
 
     def __getattr__(self, name):
-        mod = _ffi.host_calls(_WORKSPACE._bufs, _WORKSPACE.get)
-        for fn in ("attn", "gather", "scatter", "add_norm", "linear", "linear_takes", "qkv", "unmask"):
-            setattr(self, fn, getattr(mod, fn))
+        if name not in self._CALLS:
+            raise AttributeError(name)
+        _ffi.lib()  # without the kernels there is nothing to fall back to
+        mod = None
+        try:
+            mod = _ffi.host_calls(_WORKSPACE._bufs, _WORKSPACE.get)
+        except Exception as exc:  # noqa: BLE001 - whatever keeps the module from loading
+            _LOG.error("native host side of the calls unavailable, they take their Python form: %s", exc)
+        for fn in self._CALLS:
+            setattr(self, fn, getattr(mod, fn) if mod is not None else _not_plain)
         return self.__dict__[name]
+
+
+def _not_plain(*args):
+    return None
 
 
 _HOST = _Host()
@@ -702,7 +720,7 @@ def _linear(x, w, w_up, bias):
 def try_linear(x: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tensor] = None,
                bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``linear`` (``gated_linear`` with ``up_weight``) where ``linear_fits`` holds, else None."""
-    done = _HOST.linear(x, weight, up_weight, bias)
+    done = _HOST.linear(x, weight, up_weight, bias) if x.is_cuda else None
     if done is None:
         ws = (weight,) if up_weight is None else (weight, up_weight)
         if linear_fits(x, *ws, bias=bias):
