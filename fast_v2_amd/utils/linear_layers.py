@@ -6,15 +6,19 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+import torch.nn.modules.module as _every_module
 
 from .. import ops
 
 
 def plain_linear(mod: nn.Module) -> bool:
     """A torch linear layer whose call is its product alone: no subclass (adapters,
-    quantised or parametrised layers), no replaced forward and no hooks to run."""
+    quantised or parametrised layers), no replaced forward and no hooks to run, the layer's
+    own or those on every module (profilers, debuggers)."""
     return (type(mod) is nn.Linear and "forward" not in mod.__dict__ and not mod._forward_hooks and
-            not mod._forward_pre_hooks and not mod._backward_hooks and not mod._backward_pre_hooks)
+            not mod._forward_pre_hooks and not mod._backward_hooks and not mod._backward_pre_hooks and
+            not _every_module._global_forward_hooks and not _every_module._global_forward_pre_hooks and
+            not _every_module._global_backward_hooks and not _every_module._global_backward_pre_hooks)
 
 
 def streams(x: torch.Tensor, *mods: nn.Module) -> bool:

@@ -2,8 +2,10 @@
 ops.qkv_rope_kv_write against torch in float64."""
 import pytest
 import torch
+import torch.nn.modules.module as every
 
 from fast_v2_amd import ops
+from fast_v2_amd.utils import linear_layers as ll
 
 pytestmark = pytest.mark.gpu
 
@@ -137,3 +139,30 @@ def test_first_calls_of_a_stream_under_capture(gpu):
             assert all(torch.equal(a, b) for a, b in zip(outs[i], want))
             assert all(torch.equal(a, b) for a, b in zip(calls(), want))
     s.synchronize()
+
+
+def _layers(dtype=torch.bfloat16):
+    g = torch.Generator(device="cuda").manual_seed(21)
+    gate, up, down = (torch.nn.Linear(k, n, bias=False, device="cuda", dtype=dtype) for k, n in
+                      ((256, 512), (256, 512), (512, 256)))
+    with torch.no_grad():
+        for m in (gate, up, down):
+            m.weight.copy_(_ints(g, *m.weight.shape, dtype=dtype) * 0.0625)
+    return gate, up, down, _ints(g, 4, 8, 256, dtype=dtype)
+
+
+def _mlp(gate, up, down, x):
+    with torch.no_grad():
+        return ll.project(down, ll.gated(gate, up, x))
+
+
+def test_a_hook_on_every_module_sees_the_layers(gpu):
+    gate, up, down, x = _layers()
+    want, seen = _mlp(gate, up, down, x), []
+    h = every.register_module_forward_hook(lambda m, a, o: seen.append(m))
+    try:
+        got = _mlp(gate, up, down, x)
+    finally:
+        h.remove()
+    assert seen == [gate, up, down]
+    torch.testing.assert_close(got, want, rtol=2.0 ** -6, atol=2.0 ** -6 * float(want.abs().max()))

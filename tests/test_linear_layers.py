@@ -1,7 +1,9 @@
 """Which linear layers the weight-streaming kernels may stand in for (no GPU needed: the
 rule refuses before any launch)."""
+import pytest
 import torch
 import torch.nn as nn
+import torch.nn.modules.module as every
 import torch.nn.utils.parametrize as parametrize
 
 from fast_v2_amd import ops
@@ -32,3 +34,18 @@ def test_project_runs_the_module_on_cpu():
     x = torch.randn(3, 64).to(torch.bfloat16)
     assert not ll.streams(x, lin) and not ops.linear_fits(x, lin.weight)
     assert torch.equal(ll.project(lin, x), lin(x))
+
+
+@pytest.mark.parametrize("register", [
+    lambda f: every.register_module_forward_hook(lambda m, a, o: f()),
+    lambda f: every.register_module_forward_pre_hook(lambda m, a: f()),
+    lambda f: every.register_module_full_backward_hook(lambda m, gi, go: f()),
+    lambda f: every.register_module_full_backward_pre_hook(lambda m, go: f())])
+def test_hooks_on_every_module_are_run(register):
+    lin = nn.Linear(64, 8)
+    h = register(lambda: None)
+    try:
+        assert not ll.plain_linear(lin)
+    finally:
+        h.remove()
+    assert ll.plain_linear(lin)
