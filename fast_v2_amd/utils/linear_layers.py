@@ -1,7 +1,8 @@
 """Linear layers of few token rows on the weight-streaming kernels.
 
 A layer is taken over only where its call is the plain product (an ``nn.Linear`` itself,
-without hooks) and ``ops.linear_fits`` holds; every other call runs the module."""
+without hooks), nothing else has a say in it (``replaceable``) and ``ops.linear_fits`` holds;
+every other call runs the module."""
 from __future__ import annotations
 
 import torch
@@ -21,16 +22,23 @@ def plain_linear(mod: nn.Module) -> bool:
             not _every_module._global_backward_hooks and not _every_module._global_backward_pre_hooks)
 
 
+def replaceable(x: torch.Tensor) -> bool:
+    """Whether a layer's call on ``x`` is, as things stand, nothing but its product: no
+    autocast to another type."""
+    return (x.is_cuda and not torch.compiler.is_compiling() and
+            (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype))
+
+
 def streams(x: torch.Tensor, *mods: nn.Module) -> bool:
     """Whether every one of ``mods`` (layers of x) runs on the weight-streaming kernels."""
-    return (x.is_cuda and not torch.compiler.is_compiling() and
+    return (replaceable(x) and
             all(plain_linear(m) and ops.linear_fits(x, m.weight, bias=m.bias) for m in mods))
 
 
 def project(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``mod(x)``. 16 x 8 rows of the 7B layout: down_proj 42 us against 99 in the library's
     GEMM."""
-    if x.is_cuda and not torch.compiler.is_compiling() and plain_linear(mod):
+    if replaceable(x) and plain_linear(mod):
         y = ops.try_linear(x, mod.weight, None, mod.bias)
         if y is not None:
             return y
@@ -40,12 +48,11 @@ def project(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
 def gated(gate: nn.Module, up: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``silu(gate(x)) * up(x)`` (modeling.py:164). 16 x 8 rows of the 7B layout: 57 us
     against 79 for the two layers and the product kernel."""
-    if (x.is_cuda and not torch.compiler.is_compiling() and gate.bias is None and up.bias is None and
-            plain_linear(gate) and plain_linear(up)):
+    if replaceable(x) and gate.bias is None and up.bias is None and plain_linear(gate) and plain_linear(up):
         y = ops.try_linear(x, gate.weight, up.weight)
         if y is not None:
             return y
     return ops.silu_mul(gate(x), up(x))
 
 
-__all__ = ["plain_linear", "streams", "project", "gated"]
+__all__ = ["plain_linear", "replaceable", "streams", "project", "gated"]

@@ -166,3 +166,14 @@ def test_a_hook_on_every_module_sees_the_layers(gpu):
         h.remove()
     assert seen == [gate, up, down]
     torch.testing.assert_close(got, want, rtol=2.0 ** -6, atol=2.0 ** -6 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("cast", [torch.float16, torch.bfloat16])
+def test_autocast_decides_the_type(gpu, cast):
+    gate, up, down, x = _layers()
+    with torch.autocast("cuda", dtype=cast):
+        got = _mlp(gate, up, down, x)
+        with torch.no_grad():
+            want = down(ops.silu_mul(gate(x), up(x)))
+    assert got.dtype == want.dtype == cast
+    torch.testing.assert_close(got, want, rtol=2.0 ** -6, atol=2.0 ** -6 * float(want.abs().max()))
