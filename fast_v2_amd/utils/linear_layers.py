@@ -8,6 +8,8 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 import torch.nn.modules.module as _every_module
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from .. import ops
 
@@ -24,8 +26,12 @@ def plain_linear(mod: nn.Module) -> bool:
 
 def replaceable(x: torch.Tensor) -> bool:
     """Whether a layer's call on ``x`` is, as things stand, nothing but its product: no
-    autocast to another type."""
-    return (x.is_cuda and not torch.compiler.is_compiling() and
+    autocast to another type, no tracing, and no mode (a FLOP counter, a tracer) that
+    expects to see it. A default device is a mode too, but concerns new tensors only."""
+    return (x.is_cuda and not torch.compiler.is_compiling() and not torch._C._len_torch_dispatch_stack() and
+            (not torch._C._len_torch_function_stack() or
+             all(type(m) is DeviceContext for m in _get_current_function_mode_stack())) and
+            torch._C._get_tracing_state() is None and
             (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype))
 
 

@@ -4,6 +4,9 @@ import pytest
 import torch
 import torch.nn.modules.module as every
 
+from torch.overrides import TorchFunctionMode
+from torch.utils.flop_counter import FlopCounterMode
+
 from fast_v2_amd import ops
 from fast_v2_amd.utils import linear_layers as ll
 
@@ -177,3 +180,24 @@ def test_autocast_decides_the_type(gpu, cast):
             want = down(ops.silu_mul(gate(x), up(x)))
     assert got.dtype == want.dtype == cast
     torch.testing.assert_close(got, want, rtol=2.0 ** -6, atol=2.0 ** -6 * float(want.abs().max()))
+
+
+class _Calls(TorchFunctionMode):
+    def __init__(self):
+        self.linear = 0
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.linear += func is torch.nn.functional.linear
+        return func(*args, **(kwargs or {}))
+
+
+def test_modes_see_the_layers(gpu):
+    gate, up, down, x = _layers()
+    with FlopCounterMode(display=False) as flops:
+        _mlp(gate, up, down, x)
+    assert flops.get_total_flops() == 2 * 32 * 3 * 256 * 512
+    with _Calls() as calls:
+        _mlp(gate, up, down, x)
+    assert calls.linear == 3
+    with torch.device("cuda"):  # a default device changes nothing
+        assert ll.replaceable(x)
