@@ -341,7 +341,10 @@ PyObject* add_norm(PyObject* const* a, Py_ssize_t n) {
   return PyTuple_Pack(2, p.o, q.o);
 }
 
+// A gradient to record, or a forward-mode tangent to carry.
 bool differentiates(std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t && t->_fw_grad(0).defined()) return true;
   if (!c10::GradMode::is_enabled()) return false;
   for (const Tensor* t : ts)
     if (t && t->requires_grad()) return true;

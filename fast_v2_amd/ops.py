@@ -30,6 +30,7 @@ import threading
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _ffi
 
@@ -663,6 +664,17 @@ def qkv_linear(x, wq, bq, wk, bk, wv, bv, head_dim: int = 128):
     return q, k, v
 
 
+def _plain_tensors(*ts: Optional[torch.Tensor]) -> bool:
+    """Whether each tensor (or None) holds its values where it says: no subclass (quantised
+    or distributed weights), no wrapper of a function transform, no pending negation, and no
+    forward-mode tangent that a kernel would drop."""
+    if any(t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.is_neg()) for t in ts):
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    return forward_ad._current_level < 0 or all(t is None or forward_ad.unpack_dual(t).tangent is None for t in ts)
+
+
 LINEAR_MAX_ROWS = 128  # token rows of ``linear`` and ``gated_linear``
 
 
@@ -675,7 +687,8 @@ def linear_fits(x: torch.Tensor, *weights: torch.Tensor, bias: Optional[torch.Te
     w = weights[0]
     if len(weights) == 1 and x.is_cuda and _HOST.linear_takes(x, w, bias):
         return True
-    if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or x.dim() < 2 or w.dim() != 2:
+    if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or x.dim() < 2 or w.dim() != 2 or \
+            not _plain_tensors(x, *weights, bias):
         return False
     n, k = w.shape
     if x.shape[-1] != k or k % 64 or not 64 <= k <= 65536 or n % 8 or not 0 < n <= 1 << 24 or \

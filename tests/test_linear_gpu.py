@@ -3,6 +3,7 @@ ops.qkv_rope_kv_write against torch in float64."""
 import pytest
 import torch
 import torch.nn.modules.module as every
+from torch.autograd import forward_ad
 
 from torch.overrides import TorchFunctionMode
 from torch.utils.flop_counter import FlopCounterMode
@@ -201,3 +202,42 @@ def test_modes_see_the_layers(gpu):
     assert calls.linear == 3
     with torch.device("cuda"):  # a default device changes nothing
         assert ll.replaceable(x)
+
+
+class _Doubled(torch.Tensor):
+    """A weight that is not stored as it reads (as quantised weights are): twice ``inner``."""
+
+    @staticmethod
+    def __new__(cls, inner):
+        t = torch.Tensor._make_wrapper_subclass(cls, inner.shape, strides=inner.stride(), dtype=inner.dtype,
+                                                device=inner.device)
+        t.inner = inner
+        return t
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        if func is torch.ops.aten.detach.default:
+            return cls(args[0].inner)
+        return func(*[a.inner * 2 if isinstance(a, cls) else a for a in args], **(kwargs or {}))
+
+
+def test_layers_on_other_tensors_run_as_modules(gpu):
+    """Weights of a tensor subclass, forward-mode tangents and vmap: what the module gives."""
+    gate, _, down, x = _layers()
+    half = down.weight.detach() * 0.5
+    ones = torch.ones(4, 8, 512, device=gpu, dtype=torch.bfloat16)
+    want = down(ones).detach()
+    down.weight = torch.nn.Parameter(_Doubled(half), requires_grad=False)
+    with torch.no_grad():
+        torch.testing.assert_close(ll.project(down, ones), want, rtol=2.0 ** -7, atol=2.0 ** -6)
+        with forward_ad.dual_level():
+            y = ll.project(gate, forward_ad.make_dual(x, torch.ones_like(x)))
+            tangent = forward_ad.unpack_dual(y).tangent
+            assert ll.project(gate, x).shape == y.shape  # no tangent: nothing to carry
+        rows = torch.vmap(lambda r: ll.project(gate, r))(x)
+    torch.testing.assert_close(tangent, gate(torch.ones_like(x)).detach(), rtol=2.0 ** -6, atol=2.0 ** -5)
+    torch.testing.assert_close(rows, gate(x).detach(), rtol=2.0 ** -6, atol=2.0 ** -5)
+    dual = None
+    with forward_ad.dual_level(), pytest.raises(RuntimeError):
+        dual = ops.linear(forward_ad.make_dual(x, torch.ones_like(x)), gate.weight.detach())
+    assert dual is None
