@@ -82,6 +82,10 @@ struct Plan {
   size_t ws_unit_off;  // split prefill: byte offset of the unit table in the (m, l) region
 };
 
+// Sub-block decode: partial slots per KV head that give each compute unit one workgroup.
+constexpr int kMinSlotRound = 32;  // at most eight KV heads: slots in whole rounds
+inline int64_t slot_round(int64_t hkv) { return (kDecodeSlotsTarget + hkv - 1) / hkv; }
+
 // Longest key range a call can read: max_seqlen, capped by the pages' capacity.
 inline int64_t plan_max_keys(const fdllm_kv_attn_desc* d) {
   return d->page_table ? std::min<int64_t>(d->max_seqlen, static_cast<int64_t>(d->max_pages) * d->page_size)
@@ -262,15 +266,24 @@ inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl, bool lean = false) {
       }
       if (d->kv_split == 0 && B <= kBalancedMaxBatch) {
         pl->chunk = 0;
-        // one workgroup per compute unit, or whole multiples of that where long sequences may
-        // need more: 16-bit 28 / 4 heads, token-major pages, 24 x 2000-12000 keys 98.6 us
-        // with 72 slots, 79.0 with 128; 40 x 2000-6000 90.4 with 80, 73.8 with 128; 48 x
-        // 2000-6000 98.0 with 96, 87.4 with 128. More rounds than needed only cost (16 x
-        // 2000-6000: 33 us with 64 slots, 43 with 128).
-        const int64_t round = (kDecodeSlotsTarget + hkv - 1) / hkv;
-        slots = std::max<int64_t>(round, (B * min_splits + round - 1) / round * round);
-        // (what the library's scratch holds without the rounding keeps fitting it)
-        if (lean || slots * hkv * 64 * (d->head_dim + 2) * 4 > kScratchSlotBytes) slots = std::max(round, B * min_splits);
+        // One workgroup per compute unit; where sequences may need more than one split each
+        // (at the cache's capacity: the host knows no lengths), whole multiples of that: a
+        // last round that is nearly empty lasts as long as a full one. More rounds than
+        // needed only cost, so the kernel uses one or two of them where the lengths it finds
+        // fit (decode_partition). 8-token steps, us: slots unrounded / rounded / and chosen:
+        //   28/4 heads, 24 x 1000-12000 keys 88.3 / 73.0 / 67.4; 48 x 2000-12011 149.8 /
+        //   136.6 / 137.6; 64 x 1000-12000 165.9 / 165.9 / 165.9 (174.9 in two rounds)
+        //   in a cache of 8192: 33 x 64-300 11.6 / 19.8 / 11.9; 40 x 500-2000 38.9 / 35.9 / 28.4
+        //   32/8 heads, cache of 12288: 24 x 300-1000 33.0 / 34.4 / 22.0
+        // Many KV heads have many small rounds and little to gain: 32/32 heads, 12 x 500-2000
+        // in a cache of 8192 64.9 with 24 slots (as is), 75.2 with 16 (two rounds).
+        const int64_t round = slot_round(hkv);
+        slots = std::max(round, B * min_splits);
+        if (min_splits > 1 && !lean && round >= kMinSlotRound) {
+          const int64_t whole = (slots + round - 1) / round * round;
+          // (what the library's scratch holds without the rounding keeps fitting it)
+          if (whole * hkv * 64 * (d->head_dim + 2) * 4 <= kScratchSlotBytes) slots = whole;
+        }
         pl->n_splits = static_cast<int>(slots);
         split_possible = slots > B;
       } else {

@@ -106,6 +106,7 @@ struct AttnParams {
   const uint16_t* vn;
   int64_t n_sb, n_ss, n_sh;
   int cap;
+  int slot_round;   // split decode, balanced partition: slots per KV head of one round of the compute units
 #if FDLLM_TIMELINE
   uint64_t* tl;  // per-workgroup phase stamps (kTimelineStamps each), or null
 #endif
@@ -845,7 +846,10 @@ __device__ __forceinline__ int active_splits(int t, int n) {
 //     count per split (>= 4) for which the splits of all sequences fit in the S
 //     slots; the slots are handed out in sequence order. The cost of one workgroup
 //     is then at most C tiles whatever the mix of lengths, where a per-sequence
-//     chunk gives the short sequences half-empty workgroups. Every workgroup
+//     chunk gives the short sequences half-empty workgroups. Where the host laid out
+//     several rounds of slots for what the cache could hold, sub-block decode uses the
+//     one or two whole rounds that hold these lengths, while that leaves its splits at most
+//     half full on average (longer ones balance better over more rounds). Every workgroup
 //     evaluates the same integer search (binary, on one wave's lanes, one lane per
 //     sequence), so all of them agree on the partition.
 template <bool PAGED, int TILE = 32>
@@ -875,12 +879,20 @@ __device__ __forceinline__ DecodePart decode_partition(const AttnParams& p, cons
   sl.seqlen = sl.qs = sl.kv_end = 0;
   if (has) sl = seq_info<PAGED>(p, ld, lane, 0);
   const int t = (sl.kv_end + TILE - 1) / TILE;
-  const int S = p.n_splits;
   // splits of a sequence for C tiles per split (an empty sequence still takes one
   // slot); the count over-estimates only where the cap of kMaxDecodeSplits bites
   auto splits_of = [&](int C) { return max(1, min(kMaxDecodeSplits, ceil_div_small(t, C))); };
   auto count = [&](int C) { return wave_sum_i32(has ? splits_of(C) : 0); };
   const int T = wave_sum_i32(t);
+  int S = p.n_splits;
+  if (TILE == 32 && p.slot_round >= kMinSlotRound && S > p.slot_round) {
+    const int fewest = ceil_div_small(count(kDecodeMaxTiles), p.slot_round) * p.slot_round;
+    if (fewest <= 2 * p.slot_round && T <= kDecodeMaxTiles / 2 * fewest) S = min(S, fewest);
+    if (static_cast<int>(blockIdx.x) >= S) {
+      dp.b = -1;
+      return dp;
+    }
+  }
   // C = ceil(T / S) is a lower bound; ceil(T / (S - B)) fits, as each sequence
   // rounds up by less than one split (the host sizes S so that C = 160 fits).
   const int nb = min(ld.B, 64);
@@ -915,7 +927,7 @@ __device__ __forceinline__ DecodePart decode_partition(const AttnParams& p, cons
   dp.n_act = __builtin_amdgcn_readlane(n_l, b);
   const int first = __builtin_amdgcn_readlane(incl, b) - dp.n_act;
   dp.split = slot - first;
-  dp.first = blockIdx.y * S + first;  // S slots per KV head
+  dp.first = blockIdx.y * p.n_splits + first;  // n_splits slots per KV head
   dp.seqlen = __builtin_amdgcn_readlane(sl.seqlen, b);
   dp.qs = __builtin_amdgcn_readlane(sl.qs, b);
   dp.kv_end = __builtin_amdgcn_readlane(sl.kv_end, b);
@@ -3717,6 +3729,7 @@ int kv_attn_launch(const fdllm_kv_attn_desc* d, const Plan& pl, void* workspace,
   p.rows_per_wg = pl.rows_per_wg;
   p.n_rb = pl.n_rb;
   p.n_splits = pl.n_splits;
+  p.slot_round = static_cast<int>(slot_round(d->num_kv_heads));
   p.chunk = pl.chunk;
   p.mask_mode = d->mask_mode;
   p.mask_block = d->mask_block > 0 ? d->mask_block : 1;

@@ -106,6 +106,9 @@ static void check_plan(const fdllm_kv_attn_desc& d, const Plan& pl) {
         CHECK(Bm <= kBalancedMaxBatch, "per-sequence partition batch: %s", describe(d));
         CHECK(pl.n_splits >= Bm * cdiv(max_t, kDecodeMaxTiles) && pl.n_splits >= cdiv(kDecodeSlotsTarget, hkv),
               "slots %d: %s", pl.n_splits, describe(d));
+        // rounded up to whole rounds at most
+        CHECK(pl.n_splits < std::max<i128>(Bm * cdiv(max_t, kDecodeMaxTiles), 1) + cdiv(kDecodeSlotsTarget, hkv),
+              "rounds %d: %s", pl.n_splits, describe(d));
         slots = pl.n_splits;
       } else {
         CHECK(pl.chunk % 32 == 0 && pl.chunk <= kSplitMaxChunk && pl.chunk >= 32, "chunk %d: %s", pl.chunk,

@@ -1003,3 +1003,27 @@ def test_unread_rows_poisoned_with_nan(gpu, case):
     assert torch.equal(outs[0], outs[1]), "rows past the visible lengths changed the output"
     if exp is not None:
         _check(outs[0], exp)
+
+
+@pytest.mark.parametrize("heads", [(28, 4), (32, 8), (8, 4), (32, 32)])
+@pytest.mark.parametrize("b,cap,lo,hi", [(33, 8192, 40, 300), (40, 8192, 500, 2000), (24, 12288, 200, 9000),
+                                         (48, 5152, 5000, 5152), (64, 5152, 1, 5152)])
+def test_split_decode_rounds_of_slots(gpu, heads, b, cap, lo, hi):
+    """Caches that could hold long sequences make the host lay out several rounds of split
+    slots; the kernel uses one, two or all of them by the lengths it finds (a sequence empty,
+    all short, all as long as one split holds, mixed). The partition does not change what is
+    computed: the general kernel's results within rounding, and the same bits when repeated."""
+    hq, hkv = heads
+    if hkv == 32 and cap > 6000:
+        b = 12
+    g = torch.Generator(device="cuda").manual_seed(b + hkv)
+    q = torch.randn(b, 8 if hq != 8 else 2, hq, 128, generator=g, device=gpu).bfloat16()
+    k, v = (torch.randn(b, cap, hkv, 128, generator=g, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+    lens = torch.randint(lo, hi + 1, (b,), generator=g, device=gpu).to(torch.int32)
+    lens[0], lens[1], lens[2] = 0, hi, lo
+    print(f"case rounds {heads} b{b} cap {cap} {lo}-{hi}", flush=True)
+    got = ops.block_attn(q, k, v, lens)
+    gen = ops.block_attn(q, k, v, lens, decode_kernel=False)
+    # probabilities (or their sum) and results are rounded to bf16 once in each
+    torch.testing.assert_close(got.float(), gen.float(), atol=1e-2, rtol=1e-2)
+    assert torch.equal(got, ops.block_attn(q, k, v, lens)) and not got[0].any()
