@@ -99,10 +99,11 @@ inline int64_t plan_max_keys(const fdllm_kv_attn_desc* d) {
 // 0.053 us per workgroup (fitted to 12-2 and 28-4 heads, 40-3000 tokens after up to 2048).
 // Lengths are taken at the cache's capacity (the host knows no others): at shorter ones the
 // kernel cuts less, never wrongly. Bounded by the library's scratch, so that calls without a
-// workspace of their own stay possible. Measured, us (start: the general kernel up to 2047
-// rows, whole ranges above): 1 x 500 tokens after 2048, 28/4 heads, 64.7 -> 40.3; 1 x 1000
-// after 1024 55.9 -> 47; 1 x 40 after 2048 29.6 -> 22.9; 12/2 heads, block-causal, 1 x 3000
-// 74.8 -> 51, 1 x 2000 50.7 -> 36; 1 x 1500 of 28/4 heads stays whole (42, two ranges 40).
+// workspace of their own stay possible. Measured, us (the general kernel up to 2047 rows,
+// whole ranges above; cache as long as the keys): 28/4 heads, 1 x 40 tokens after 512 25.7 ->
+// 17.3, 1 x 157 in a cache of 4096 36.9 -> 15.5; 12/2, block-causal, 1 x 3000 67.5 -> 49.0,
+// 1 x 2048 48.0 -> 34.4; 16/16, 1 x 1536 83.9 -> 41.2 (1 x 1000, where the fit sees no gain in
+// cutting: 34.1 -> 35.8).
 inline void plan_ring_chunk(const fdllm_kv_attn_desc* d, int R, int64_t max_len, int64_t* splits, int64_t* chunk_tiles) {
   const int G = d->num_q_heads / d->num_kv_heads;
   const int n_rb = (R + 255) / 256;
@@ -393,7 +394,11 @@ inline int make_plan(const fdllm_kv_attn_desc* d, Plan* pl, bool lean = false) {
                           d->v_stride_slot < (1 << 24) && (pl->R + 255) / 256 < 65536 &&
                           (d->k_new == nullptr || d->new_stride_s >= 128);
   int64_t ring_splits = 1, ring_tiles = std::max<int64_t>(1, (max_len + kKT - 1) / kKT);
-  if (ring_shape && !lean) plan_ring_chunk(d, pl->R, max_len, &ring_splits, &ring_tiles);
+  // (2048 rows and more: only where the cache holds little but the prompt's own keys. In one
+  // with room for more the host cannot tell a short prompt from a long prefix, and a short one
+  // pays for the merge's launch and its partials: 28/4 heads, 1 x 500 tokens in a cache of
+  // 1024 18.9 us whole, 23.1 with ranges; 2 x 500 of 4096 19.8, 22.7)
+  if (ring_shape && !lean && (!prefill_shape || max_len - d->q_len < kKT)) plan_ring_chunk(d, pl->R, max_len, &ring_splits, &ring_tiles);
   pl->ring = ring_shape && (ring_splits > 1 || !prefill_shape);
   if (prefill_shape && !pl->ring) {
     pl->kind = kPlanPrefill;

@@ -56,10 +56,10 @@ def _ref(q, k, v, table, lens, starts, mode, block=32):
 
 
 # rows per KV head: 259 (two row blocks), 1099, 2037 / 2051 (around the whole-range form's
-# start), 3500; key ranges where the capacity is long; visible lengths at, below and far
+# start), 3500, 7218 that fill the cache (key ranges); key ranges where the capacity is long; visible lengths at, below and far
 # below the capacity (one sequence empty of keys to range over)
 SHAPES = [(1, 37, (28, 4), 37), (2, 157, (28, 4), 157), (1, 291, (28, 4), 1500), (1, 293, (28, 4), 293),
-          (1, 500, (28, 4), 1203), (1, 300, (12, 2), 2048), (3, 70, (12, 2), 700), (1, 129, (2, 1), 4096)]
+          (1, 500, (28, 4), 1203), (1, 300, (12, 2), 2048), (1, 1203, (12, 2), 1203), (3, 70, (12, 2), 700), (1, 129, (2, 1), 4096)]
 
 
 @pytest.mark.parametrize("b,sq,heads,cap", SHAPES)
@@ -96,9 +96,11 @@ def test_prompt_query_starts_and_empty_rows(gpu, starts):
             torch.testing.assert_close(got.double(), _ref(q, k, v, table, lens, starts, mode), atol=1e-2, rtol=1e-2)
 
 
-def test_prompt_graph_replay(gpu):
-    """Ranges and their merge under graph replay with eager calls in between."""
-    q, k, v, table, kn, vn = _case(1, 500, (28, 4), 1203, "contiguous", torch.bfloat16, 9)
+@pytest.mark.parametrize("sq,heads", [(500, (28, 4)), (1203, (12, 2)), (280, (28, 4))])
+def test_prompt_graph_replay(gpu, sq, heads):
+    """A prompt whole (3500 rows in a cache with room for more) and its ranges with their merge
+    (7218 rows that fill the cache; 1960 rows) under graph replay, eager calls in between."""
+    q, k, v, table, kn, vn = _case(1, sq, heads, 1203, "contiguous", torch.bfloat16, 9)
     seqlens = torch.tensor([1203], dtype=torch.int32, device="cuda")
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
@@ -129,11 +131,11 @@ def _c_call(q, k, v, seqlens, mode, ws_bytes):
 def test_workspace_of_a_plan_without_ranges(gpu):
     """A prompt without a workspace runs whole; a decode call with the slots it cannot do
     without runs on those; less is refused."""
-    q, k, v, _, _, _ = _case(1, 500, (28, 4), 1203, "contiguous", torch.bfloat16, 3)
+    q, k, v, _, _, _ = _case(1, 1203, (12, 2), 1203, "contiguous", torch.bfloat16, 3)
     lens = torch.tensor([1203], dtype=torch.int32, device="cuda")
     rc, out = _c_call(q, k, v, lens, _ffi.MASK_CAUSAL, 0)
     assert rc == _ffi.FDLLM_OK
-    torch.testing.assert_close(out.double(), _ref(q, k, v, None, [1203], [703], _ffi.MASK_CAUSAL), atol=1e-2, rtol=1e-2)
+    torch.testing.assert_close(out.double(), _ref(q, k, v, None, [1203], [0], _ffi.MASK_CAUSAL), atol=1e-2, rtol=1e-2)
 
     q, k, v, _, _, _ = _case(33, 2, (8, 4), 5152, "contiguous", torch.bfloat16, 4)  # two splits each: 66 slots, or 128
     lens = torch.tensor([40 * i + 5 for i in range(33)], dtype=torch.int32, device="cuda")
@@ -151,7 +153,7 @@ def test_calls_of_two_threads_on_one_stream(gpu):
     def call(b, sq, n, seed, mode):
         q, k, v, _, _, _ = _case(b, sq, (28, 4), n, "contiguous", torch.bfloat16, seed)
         return q, k, v, torch.full((b,), n, dtype=torch.int32, device="cuda"), mode
-    calls = [call(1, 300, 2048, 1, _ffi.MASK_CAUSAL), call(4, 32, 1500, 2, _ffi.MASK_SEQLEN),
+    calls = [call(1, 280, 2048, 1, _ffi.MASK_CAUSAL), call(4, 32, 1500, 2, _ffi.MASK_SEQLEN),
              call(4, 8, 1500, 3, _ffi.MASK_SEQLEN)]
     run = [lambda c=c: ops.block_attn(*c[:4], mask_mode=c[4]) for c in calls]
     want = [f() for f in run]
