@@ -682,8 +682,7 @@ def linear_fits(x: torch.Tensor, *weights: torch.Tensor, bias: Optional[torch.Te
     """Whether ``linear`` (``gated_linear`` with two weights) takes this layer: at most 128
     rows of a 16-bit type, in_features a multiple of 64 (at most 65536), out_features a
     multiple of 8, contiguous aligned weights on x's device, nothing to differentiate.
-    Below 128 rows a layer is bound by reading its weights once; above, by the products,
-    where the library's tiles are the better ones."""
+    Whether it is the faster one depends on the sizes (``utils.linear_layers.pays``)."""
     w = weights[0]
     if len(weights) == 1 and x.is_cuda and _HOST.linear_takes(x, w, bias):
         return True

@@ -148,11 +148,12 @@ def test_first_calls_of_a_stream_under_capture(gpu):
 def _layers(dtype=torch.bfloat16):
     g = torch.Generator(device="cuda").manual_seed(21)
     gate, up, down = (torch.nn.Linear(k, n, bias=False, device="cuda", dtype=dtype) for k, n in
-                      ((256, 512), (256, 512), (512, 256)))
+                      ((1024, 2048), (1024, 2048), (2048, 1024)))
     with torch.no_grad():
         for m in (gate, up, down):
             m.weight.copy_(_ints(g, *m.weight.shape, dtype=dtype) * 0.0625)
-    return gate, up, down, _ints(g, 4, 8, 256, dtype=dtype)
+    assert ll.pays(32, 1024, 2048, False)  # else the module runs anyway
+    return gate, up, down, _ints(g, 4, 8, 1024, dtype=dtype)
 
 
 def _mlp(gate, up, down, x):
@@ -196,7 +197,7 @@ def test_modes_see_the_layers(gpu):
     gate, up, down, x = _layers()
     with FlopCounterMode(display=False) as flops:
         _mlp(gate, up, down, x)
-    assert flops.get_total_flops() == 2 * 32 * 3 * 256 * 512
+    assert flops.get_total_flops() == 2 * 32 * 3 * 1024 * 2048
     with _Calls() as calls:
         _mlp(gate, up, down, x)
     assert calls.linear == 3
@@ -225,7 +226,7 @@ def test_layers_on_other_tensors_run_as_modules(gpu):
     """Weights of a tensor subclass, forward-mode tangents and vmap: what the module gives."""
     gate, _, down, x = _layers()
     half = down.weight.detach() * 0.5
-    ones = torch.ones(4, 8, 512, device=gpu, dtype=torch.bfloat16)
+    ones = torch.ones(4, 8, 2048, device=gpu, dtype=torch.bfloat16)
     want = down(ones).detach()
     down.weight = torch.nn.Parameter(_Doubled(half), requires_grad=False)
     with torch.no_grad():
