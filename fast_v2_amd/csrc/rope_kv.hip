@@ -492,13 +492,22 @@ bool qkv_empty(const fdllm_qkv_rope_desc& d) {
   return d.rope.batch == 0 || d.rope.seq_len == 0 || d.rope.num_q_heads + d.rope.num_kv_heads == 0;
 }
 
-// 64-row weight tiles whose partial sums have counters and whose rows stay within 32 bits
-bool qkv_skinny(const fdllm_qkv_rope_desc& d) {
+// few rows, and tiles whose counts stay within 32 bits
+bool qkv_few(const fdllm_qkv_rope_desc& d) {
   return static_cast<int64_t>(d.rope.batch) * d.rope.seq_len <= kSkinnyMaxRows &&
          static_cast<int64_t>(d.rope.num_q_heads) + 2 * static_cast<int64_t>(d.rope.num_kv_heads) <= 65536;
 }
 
-// plain: cos / sin may be absent together where the few-row form runs
+// ... on the weight-streaming kernel (projection calls, us, tiles above / here): 28/4 heads,
+// hidden 3584, 8 rows 25.0 / 12.3, 128 rows 29.5 / 18.7; 12/2, 1536 13.3 / 8.6, 16.6 / 14.9;
+// 64/8, 8192 56.5 / 39.6, 63.0 / 62.3. Not many rows of short weights, where K cannot be cut
+// far and the tiles' larger share per workgroup wins: 4/1, 512, 128 rows 8.1 / 9.3, 16/16,
+// 1024 12.4 / 12.9 (64 rows 7.3 / 7.4, 11.0 / 10.4).
+bool qkv_skinny(const fdllm_qkv_rope_desc& d) {
+  return qkv_few(d) && (static_cast<int64_t>(d.rope.batch) * d.rope.seq_len <= 64 || d.hidden > 1024);
+}
+
+// plain: cos / sin may be absent together for few rows
 int check_qkv(const fdllm_qkv_rope_desc* d, bool plain) {
   FDLLM_CHECK_ARG(d != nullptr, "fdllm_qkv_rope_kv_write: null descriptor");
   const fdllm_rope_kv_desc& r = d->rope;
@@ -516,7 +525,7 @@ int check_qkv(const fdllm_qkv_rope_desc* d, bool plain) {
   const int64_t T = static_cast<int64_t>(r.batch) * r.seq_len;
   FDLLM_CHECK_ARG(T < (int64_t{1} << 30), "fdllm_qkv_rope_kv_write: too many tokens");
   FDLLM_CHECK_ARG(d->x && d->wq && d->wk && d->wv && r.q_out, "fdllm_qkv_rope_kv_write: null pointer");
-  FDLLM_CHECK_ARG(r.cos && r.sin || plain && !r.cos && !r.sin && qkv_skinny(*d), "fdllm_qkv_rope_kv_write: null cos / sin");
+  FDLLM_CHECK_ARG(r.cos && r.sin || plain && !r.cos && !r.sin && qkv_few(*d), "fdllm_qkv_rope_kv_write: null cos / sin");
   FDLLM_CHECK_ARG((r.k_out == nullptr) == (r.v_out == nullptr) && (r.k_cache == nullptr) == (r.v_cache == nullptr) &&
                       (r.k_block == nullptr) == (r.v_block == nullptr),
                   "fdllm_qkv_rope_kv_write: k and v destinations must be given together");
@@ -559,7 +568,6 @@ extern "C" int fdllm_qkv_rope_kv_write_ws(const fdllm_qkv_rope_desc* d, void* wo
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t T = static_cast<int64_t>(r.batch) * r.seq_len;
   if (qkv_skinny(*d)) {
-    // 16 x 8 rows of the 7B layout: 26.5 us on the tiles below (72 workgroups), 18.1 here
     SkinnyArgs k = skinny_qkv_plan(*d, workspace != nullptr);
     const size_t need = skinny_workspace(k, kSkinnyBN);
     FDLLM_CHECK_ARG(workspace == nullptr || (workspace_bytes >= need && al16(workspace)),
@@ -582,7 +590,7 @@ extern "C" int fdllm_qkv_rope_kv_write_ws(const fdllm_qkv_rope_desc* d, void* wo
   const int heads = r.num_q_heads + 2 * r.num_kv_heads;
   FDLLM_CHECK_ARG(static_cast<int64_t>(a.n_mt) * heads * 2 < (int64_t{1} << 30), "fdllm_qkv_rope_kv_write: too many tiles");
   // Whole-head tiles while they give the compute units more than half a workgroup each;
-  // with fewer (few heads), half-head tiles, twice as many workgroups each streaming 3/4 of
+  // with fewer (few heads or rows), half-head tiles, twice as many workgroups each streaming 3/4 of
   // the bytes (36 whole-head tiles of the 7B layout: 29 against 41 us; at 512 rows the
   // half-head form, 288 workgroups for 256 compute units, took 55 against 40 us).
   const bool half_head = a.n_mt * heads <= 128;

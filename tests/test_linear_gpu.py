@@ -85,20 +85,21 @@ def test_linear_refuses(gpu, bad):
         ops.linear(x, w)
 
 
-@pytest.mark.parametrize("rows", [(1, 1), (4, 8), (5, 13), (4, 32)])
-def test_qkv_linear_is_the_fused_kernels_projection(gpu, rows):
+@pytest.mark.parametrize("hidden", [1536, 1024, 512])  # the last two on the other kernel from 65 rows
+@pytest.mark.parametrize("rows", [(1, 1), (4, 8), (8, 8), (5, 13), (4, 32)])
+def test_qkv_linear_is_the_fused_kernels_projection(gpu, rows, hidden):
     """Plain projections, and the ones that qkv_rope_kv_write rotates (v rows as they are)."""
     g = torch.Generator(device="cuda").manual_seed(11)
     b, s = rows
     dt = torch.bfloat16
-    x = torch.randn(b, s, 1536, generator=g, device="cuda").to(dt)
-    w = [(torch.randn(n, 1536, generator=g, device="cuda") * 0.02).to(dt) for n in (768, 256, 256)]
+    x = torch.randn(b, s, hidden, generator=g, device="cuda").to(dt)
+    w = [(torch.randn(n, hidden, generator=g, device="cuda") * 0.02).to(dt) for n in (768, 256, 256)]
     bias = [torch.randn(t.shape[0], generator=g, device="cuda").to(dt) for t in w]
     args = [t for pair in zip(w, bias) for t in pair]
     q, k, v = ops.qkv_linear(x, *args)
     for got, wt, bt in zip((q, k, v), w, bias):
         want = x.double() @ wt.double().t().contiguous() + bt.double()
-        # one rounding to bf16 (half of 2^-7 of the value) and fp32 sums of 1536 products
+        # one rounding to bf16 (half of 2^-7 of the value) and fp32 sums of at most 1536 products
         torch.testing.assert_close(got.reshape(b, s, -1).double(), want, rtol=2.0 ** -8 + 2e-5, atol=2e-4)
     cos, sin = (torch.randn(1, s, 128, generator=g, device="cuda").to(dt) for _ in range(2))
     q_rot, (k_rot, v_out) = ops.qkv_rope_kv_write(x, *args, cos, sin, kv_out=True)
