@@ -52,8 +52,11 @@ def pays(rows: int, n: int, k: int, gated: bool) -> bool:
     n = 8192: with longer k (28672: 0.58-1.02), not at 8192 x 8192 (0.95-1.42).
     n up to 16384, not cut over k: up to 16 rows (0.78-0.99; 0.88-1.07 above).
     n from 16384 (lm_head): up to 48 rows where the tiles are one round (0.71-0.99; 0.73-1.18
-    above) or nearly fill their last one (18944, 20480, 152064 columns: 0.41-0.97; 16384,
-    51200, 128256, which do not: 0.99-1.14)."""
+    above), cut over k only if they nearly fill it (18944, 20480 columns: 0.41-0.97; 16384:
+    1.02-1.14). Several rounds at any row count if the last is nearly full (151936 x 896 and
+    x 1536: 0.48-0.95; 152064 x 3584 0.72-1.04 by itself, and a two-layer step is shorter by 5-19
+    us at every count, 581 against 600 at 128 rows); not 51200 and 128256, which it is not:
+    0.99-1.22."""
     wide = n * (2 if gated else 1) >= 16384
     per = (160 if wide else 64) // (2 if gated else 1)
     tiles = -(-n // per)
@@ -64,7 +67,7 @@ def pays(rows: int, n: int, k: int, gated: bool) -> bool:
     if not wide:
         return rows <= 16
     wgs = tiles * (2 if tiles <= 128 else 1)
-    return rows <= 48 and (128 < tiles <= 256 or wgs >= 0.9 * 256 * -(-wgs // 256))
+    return (rows <= 48 or tiles > 256) and (128 < tiles <= 256 or wgs >= 0.9 * 256 * -(-wgs // 256))
 
 
 def _rows(x: torch.Tensor) -> int:

@@ -55,7 +55,7 @@ def test_hooks_on_every_module_are_run(register):
     (18944, 3584, True, 128), (8960, 1536, True, 128), (28672, 8192, True, 32), (3584, 18944, False, 128),
     (1536, 8960, False, 128), (2048, 2048, False, 64), (896, 896, False, 0), (8192, 8192, False, 0),
     (8192, 28672, False, 128), (11008, 4096, False, 16), (16384, 4096, False, 0), (32000, 4096, False, 48),
-    (151936, 1536, False, 48), (152064, 3584, False, 48), (128256, 4096, False, 0), (51200, 2048, False, 0)])
+    (151936, 1536, False, 128), (152064, 3584, False, 128), (128256, 4096, False, 0), (51200, 2048, False, 0)])
 def test_layers_that_pay(n, k, gated, most):
     """The largest row count at which the kernel stands in for a layer."""
     assert [m for m in range(1, 129) if ll.pays(m, n, k, gated)] == list(range(1, most + 1))
