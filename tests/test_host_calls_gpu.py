@@ -12,6 +12,26 @@ from fast_v2_amd import _ffi, ops
 pytestmark = pytest.mark.gpu
 
 
+class _Recorded:
+    """The native module's functions; notes which calls they left to Python."""
+
+    def __init__(self, host):
+        self.host, self.native, self.python = host, set(), set()
+
+    def __getattr__(self, name):
+        fn = getattr(self.host, name)
+
+        def call(*a):
+            try:
+                out = fn(*a)
+            except Exception:  # refused by the C ABI: the native call got that far
+                self.native.add(name)
+                raise
+            (self.python if out is None else self.native).add(name)
+            return out
+        return call
+
+
 class _Off:
     """Every call "not in the plain form"."""
 
@@ -29,12 +49,25 @@ def _python():
         ops._HOST = saved
 
 
-def _both(make):
+@contextlib.contextmanager
+def _native(python):
+    """Only the calls named in ``python`` may be left to the Python form."""
+    saved = ops._HOST
+    ops._HOST = _Recorded(saved)
+    try:
+        yield
+        assert ops._HOST.python == set(python), (ops._HOST.native, ops._HOST.python)
+        assert not ops._HOST.native & set(python)
+    finally:
+        ops._HOST = saved
+
+
+def _both(make, python=()):
     """The call's outputs and its tensors afterwards, natively and in Python."""
     res = []
     for off in (False, True):
         fn, state = make()
-        with _python() if off else contextlib.nullcontext():
+        with _python() if off else _native(python):
             try:
                 out = fn()
             except Exception as exc:  # noqa: BLE001 - compared below
@@ -102,7 +135,8 @@ def _attn(form):
                                   "q_start", "scale", "heads", "types", "cpu_lens", "mask", "grad", "empty"])
 def test_attention(gpu, form):
     print(f"case attention {form}", flush=True)
-    a, b = _both(_attn(form))
+    left = form in ("q_strided", "int64_lens", "write_strides", "heads", "types", "cpu_lens")
+    a, b = _both(_attn(form), ("attn",) if left else ())
     _same(a, b)
 
 
@@ -137,7 +171,9 @@ def test_gather_add_scatter(gpu, form):
             ops.scatter_rows(s, idx, cache)
             return normed, got, s, n
         return fn, (cache, cur)
-    _same(*_both(make))
+    left = {"int32": ("gather", "scatter"), "columns": ("gather", "scatter"), "no_weight": ("gather",),
+            "weight_size": ("gather",), "strided": ("gather",)}
+    _same(*_both(make, left.get(form, ())))
 
 
 @pytest.mark.parametrize("form", ["plain", "offset", "no_block", "strided_x", "cos2d", "batch_cos", "no_bias", "types", "shape"])
@@ -164,7 +200,7 @@ def test_projections(gpu, form):
         elif form == "shape":
             kc = kc[:, :, :, :64]
         return (lambda: ops.qkv_rope_kv_write(x, w[0], b[0], w[1], b[1], w[2], b[2], cs, cs, kc, vc, **kw)), (kc, vc, kb, vb)
-    _same(*_both(make))
+    _same(*_both(make, ("qkv",) if form in ("cos2d", "types", "shape") else ()))
 
 
 @pytest.mark.parametrize("form", ["plain", "stop", "no_finished", "bytes", "strided", "int32_tokens"])
@@ -191,7 +227,7 @@ def test_unmask(gpu, form):
 def test_linear_strided_and_grad(gpu):
     w = _rnd(1, 64, 128)
     for x in (_rnd(2, 4, 8, 128), _rnd(2, 4, 16, 128)[:, 8:], _rnd(2, 8, 256)[:, 128:]):
-        _same(*_both(lambda: ((lambda: ops.linear(x, w)), ())))
+        _same(*_both(lambda: ((lambda: ops.linear(x, w)), ()), () if x.is_contiguous() else ("linear",)))
     p = torch.nn.Parameter(w)
     with torch.no_grad():
         assert torch.equal(ops.linear(_rnd(2, 8, 128), p), ops.linear(_rnd(2, 8, 128), w))
@@ -240,3 +276,20 @@ def test_streams_and_threads(gpu):
         [t.start() for t in threads]
         [t.join() for t in threads]
         assert bad == [0, 0]
+
+
+def test_inference_mode_and_the_callers_scratch(gpu):
+    with torch.inference_mode():
+        _same(*_both(_attn("plain")))
+        lg = _rnd(1, 3, 8, 4096) * 6
+        kept = ops.UnmaskScratch(3, 8, lg.device)
+
+        def make():
+            tok = torch.full((3, 8), 4095, dtype=torch.int64, device="cuda")
+
+            def fn():
+                sc = ops.unmask_step(lg, tok, 4095, 0.9, scratch=kept)
+                assert sc is kept
+                return sc.row_tok.clone(), sc.row_conf.clone(), sc.counts.clone()
+            return fn, tok
+        _same(*_both(make))

@@ -1,5 +1,7 @@
 """ops.linear / ops.gated_linear (fdllm_linear) and the few-row form of
 ops.qkv_rope_kv_write against torch in float64."""
+import ctypes
+
 import pytest
 import torch
 import torch.nn.modules.module as every
@@ -8,7 +10,7 @@ from torch.autograd import forward_ad
 from torch.overrides import TorchFunctionMode
 from torch.utils.flop_counter import FlopCounterMode
 
-from fast_v2_amd import ops
+from fast_v2_amd import _ffi, ops
 from fast_v2_amd.utils import linear_layers as ll
 
 pytestmark = pytest.mark.gpu
@@ -21,9 +23,12 @@ def _ints(gen, *shape, dtype):
 
 
 # rows at the edges of the 16-row MFMA tile counts; columns and K where a layer is one
-# tile, a partial last tile, tiles cut evenly (<= 128 tiles) and ranges that cross tiles
+# tile, a partial last tile, tiles cut evenly (<= 128 tiles) and ranges that cross tiles;
+# wide tiles (from 16384 columns) with K steps beyond the ring's slots, so that slots are
+# refilled: in two ranges (103, 105 tiles), in one (129)
 @pytest.mark.parametrize("m", [1, 16, 17, 33, 64, 65, 128])
-@pytest.mark.parametrize("n,k", [(8, 64), (72, 576), (200, 4096), (8320, 1088), (16648, 192)])
+@pytest.mark.parametrize("n,k", [(8, 64), (72, 576), (200, 4096), (8320, 1088), (16648, 192), (16392, 1088), (16648, 1088),
+                                 (20488, 1024)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_linear_exact(gpu, m, n, k, dtype):
     print(f"case linear {m}x{n}x{k} {dtype}", flush=True)
@@ -45,8 +50,8 @@ def test_linear_strided_rows(gpu):
         assert torch.equal(ops.linear(x, w), (x.double() @ w.double().t().contiguous()).float().to(x.dtype))
 
 
-@pytest.mark.parametrize("m", [1, 31, 128])
-@pytest.mark.parametrize("n,k", [(8, 64), (104, 1536), (4360, 1088)])
+@pytest.mark.parametrize("m", [1, 31, 33, 64, 65, 128])
+@pytest.mark.parametrize("n,k", [(8, 64), (104, 1536), (4360, 1088), (8200, 1088), (10248, 512), (18952, 1088)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gated_linear(gpu, m, n, k, dtype):
     print(f"case gated {m}x{n}x{k} {dtype}", flush=True)
@@ -243,3 +248,33 @@ def test_layers_on_other_tensors_run_as_modules(gpu):
     with forward_ad.dual_level(), pytest.raises(RuntimeError):
         dual = ops.linear(forward_ad.make_dual(x, torch.ones_like(x)), gate.weight.detach())
     assert dual is None
+
+
+@pytest.mark.parametrize("m,n,k,gated", [(1, 200, 4096, False), (65, 200, 4096, False), (128, 4360, 1088, True),
+                                         (33, 16392, 1088, False)])
+def test_linear_without_a_workspace(gpu, m, n, k, gated):
+    """fdllm_linear with no workspace: one K range, the same sums."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    dt = torch.bfloat16
+    x, w, u = _ints(g, m, k, dtype=dt), _ints(g, n, k, dtype=dt), _ints(g, n, k, dtype=dt)
+    w = w * 0.015625 if gated else w
+    out = torch.empty(m, n, dtype=dt, device=gpu)
+    _ffi.check(_ffi.lib().fdllm_linear(x.data_ptr(), k, w.data_ptr(), u.data_ptr() if gated else None, None,
+                                       out.data_ptr(), m, n, k, _ffi.dtype_code(dt), None, 0, _ffi.stream_ptr(gpu)),
+               "fdllm_linear")
+    assert torch.equal(out, ops.gated_linear(x, w, u) if gated else ops.linear(x, w))
+
+
+@pytest.mark.parametrize("rows,hidden", [((4, 8), 1536), ((4, 32), 1536), ((4, 32), 1024), ((5, 32), 1536)])
+def test_projections_without_a_workspace(gpu, rows, hidden):
+    """fdllm_qkv_rope_kv_write takes none: whole numbers, whose sums are exact in any order."""
+    g = torch.Generator(device="cuda").manual_seed(hidden)
+    (b, s), dt = rows, torch.bfloat16
+    x, w = _ints(g, b, s, hidden, dtype=dt), [_ints(g, n, hidden, dtype=dt) for n in (768, 256, 256)]
+    cs = torch.randn(1, s, 128, generator=g, device="cuda").to(dt)
+    want, (wk, wv) = ops.qkv_rope_kv_write(x, w[0], None, w[1], None, w[2], None, cs, cs, kv_out=True)
+    d, dims, keep = ops._qkv_desc(x, w[0], None, w[1], None, w[2], None, 128)
+    q, (k, v), kept = ops._rope_dest_desc(d.rope, *dims[:5], dt, gpu, cs, cs, None, None, None, 0, None, None, 0, None,
+                                          True)
+    _ffi.check(_ffi.lib().fdllm_qkv_rope_kv_write(ctypes.byref(d), _ffi.stream_ptr(gpu)), "fdllm_qkv_rope_kv_write")
+    assert torch.equal(q, want) and torch.equal(k, wk) and torch.equal(v, wv)

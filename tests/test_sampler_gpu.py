@@ -205,3 +205,19 @@ def test_sums_of_exponentials_carry_no_bias(gpu, dtype):
     err = got[..., 1].double() / torch.exp(r - top[..., None]).sum(dim=-1) - 1
     print(f"rms {err.pow(2).mean().sqrt():.2e} mean {err.mean():.2e}")
     assert abs(float(err.mean())) < 2e-8 and float(err.abs().max()) < 5e-7
+
+
+@pytest.mark.parametrize("V", [1, 1000, 4099, 32001])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_step_without_a_workspace(gpu, V, dtype):
+    """The two forms of the step choose the same tokens; confidences within one ulp of the
+    logits' type (the sums' order differs)."""
+    g = torch.Generator().manual_seed(V)
+    raw = (torch.randn(5, 6, V, generator=g) * 2).to(dtype).to(gpu)
+    x = torch.full((5, 6), V + 5, dtype=torch.int64, device=gpu)
+    y = x.clone()
+    a = ops.unmask_step(raw, x, V + 5, 0.4, shift=0)
+    b = _step_without_workspace(raw, y, V + 5, 0.4)
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    assert torch.equal(a.row_tok, b.row_tok) and torch.equal(x, y) and torch.equal(a.counts, b.counts)
+    torch.testing.assert_close(a.row_conf, b.row_conf, atol=0, rtol=ulp)
