@@ -55,7 +55,7 @@ __device__ __forceinline__ float rnd16(float x) {
 // (max, first index, sum of exp(x - max)) of two partial states
 __device__ __forceinline__ void combine(float& m, int& idx, float& s, float m2, int idx2, float s2) {
   if (m2 > m || (m2 == m && idx2 < idx)) {
-    const float sc = m == -INFINITY ? 0.f : expf(m - m2);
+    const float sc = m == -INFINITY ? 0.f : expf(m - m2);  // (a NaN sum is kept)
     s = s * sc + s2;
     m = m2;
     idx = idx2;
@@ -81,7 +81,8 @@ __global__ __launch_bounds__(kThreads) void unmask_rows_kernel(const UnmaskArgs 
   const uint16_t* row = a.logits + b * a.lg_sb + static_cast<int64_t>(r) * a.lg_sr;
   const bool vec = (a.V % 8 == 0) && ((reinterpret_cast<uintptr_t>(row) & 15u) == 0);
 
-  // ---- pass 1: max, its first index, sum of exp(x - max)
+  // ---- pass 1: max, its first index, sum of exp(x - max). While a thread has seen nothing
+  // above -inf its sum is 0, or NaN after a NaN logit, which then stays
   float m = -INFINITY, s = 0.f;
   int idx = 0x7fffffff;
   if (vec) {
@@ -103,22 +104,23 @@ __global__ __launch_bounds__(kThreads) void unmask_rows_kernel(const UnmaskArgs 
           iv = j;
         }
       if (mv > m) {  // a strictly larger value: indices grow, so the first one is kept
-        s = m == -INFINITY ? 0.f : s * expf(m - mv);
+        if (m != -INFINITY) s *= expf(m - mv);
         m = mv;
         idx = 8 * v + iv;
       }
+      const float ref = m == -INFINITY ? 0.f : m;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s += expf(x[j] - m);
+      for (int j = 0; j < 8; ++j) s += expf(x[j] - ref);
     }
   } else {
     for (int v = tid; v < a.V; v += kThreads) {
       const float x = Elt<T>::lo(row[v]);
       if (x > m) {
-        s = m == -INFINITY ? 0.f : s * expf(m - x);
+        if (m != -INFINITY) s *= expf(m - x);
         m = x;
         idx = v;
       }
-      s += expf(x - m);
+      s += expf(x - (m == -INFINITY ? 0.f : m));
     }
   }
   // wave then workgroup reduction
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(kThreads) void unmask_rows_kernel(const UnmaskArgs 
   }
   __syncthreads();
   m = s_fin[0];
-  s = s_fin[1];
+  s = m == -INFINITY ? __builtin_nanf("") : s_fin[1];  // no finite logit: no probability
   // ---- pass 2: first index whose rounded probability equals the rounded maximum
   const float pmax = rnd16<T>(1.f / s);
   const float lo_cut = m - 0.0078125f;  // exp(x - m) < 1 - 2^-8 below it: no tie possible

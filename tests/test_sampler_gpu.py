@@ -167,7 +167,7 @@ def test_rows_without_a_finite_probability(gpu, V, workspace):
     raw[1] = float("nan")
     raw[1, 3] = float("-inf")
     raw[2, 0, 7] = float("inf")
-    raw[2, 1, 9] = float("nan") if workspace else float("inf")
+    raw[2, 1, 9] = float("nan")
     x = torch.full((B, L), V, dtype=torch.int64, device=gpu)
     rawg = raw.to(gpu)
     print(f"case non-finite rows V={V} workspace={workspace}", flush=True)
@@ -211,9 +211,10 @@ def test_sums_of_exponentials_carry_no_bias(gpu, dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_step_without_a_workspace(gpu, V, dtype):
     """The two forms of the step choose the same tokens; confidences within one ulp of the
-    logits' type (the sums' order differs)."""
+    logits' type (the sums' order differs); excluded tokens (-inf) take no part."""
     g = torch.Generator().manual_seed(V)
     raw = (torch.randn(5, 6, V, generator=g) * 2).to(dtype).to(gpu)
+    raw[1, :, :V // 2] = raw[2, 3, V // 2 + 1:] = float("-inf")  # most of a row may be excluded
     x = torch.full((5, 6), V + 5, dtype=torch.int64, device=gpu)
     y = x.clone()
     a = ops.unmask_step(raw, x, V + 5, 0.4, shift=0)
