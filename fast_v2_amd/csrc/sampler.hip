@@ -7,18 +7,18 @@
 // equals the rounded maximum probability (torch.argmax over the rounded softmax returns
 // the first of equal values); only logits within 2^-7 of the maximum can tie.
 //
-// With a workspace (fdllm_unmask_step_ws) a row is cut into chunks of kChunk logits, one
-// workgroup each: unmask_chunks_kernel reads its chunk once into registers and writes
+// With a workspace (fdllm_unmask_step_ws) a long row is cut into chunks of kChunk logits, one
+// workgroup each (unmask_cut says from where): unmask_chunks_kernel reads its chunk once into registers and writes
 // (max, its first index, sum of exp(l - max), whether a smaller logit could still tie);
 // unmask_finish_kernel, one workgroup per sequence, folds the chunks of each position,
 // re-reads only the chunks in which a tie is possible, and applies the unmask rule.
 // What bounds it: the one read of the logits. 16 x 8 positions of 152064 bf16 logits
-// (38.9 MB): 10.9 us (3.6 TB/s) + 5.0 us for the finish, against 50.0 us (128 workgroups, an
+// (38.9 MB): 9.8 us (4.0 TB/s) + 4.9 us for the finish, against 50.0 us (128 workgroups, an
 // online rescale chain per thread and the second read) + 4.4 us for the form below.
 // 8192 logits per workgroup (four 16-byte loads per thread in flight, 2432 workgroups)
 // keep every compute unit at eight workgroups.
 //
-// Without one (fdllm_unmask_step): unmask_rows_kernel, one workgroup per position, reads
+// Without one (fdllm_unmask_step), and for short rows: unmask_rows_kernel, one workgroup per position, reads
 // its row twice (pass 1: running maximum, its first index and the online sum; pass 2: the
 // first tie), then unmask_select_kernel, one wave per sequence, applies the rule.
 #include <math.h>
@@ -433,6 +433,17 @@ __global__ __launch_bounds__(kFinishThreads) void unmask_finish_kernel(const Unm
   }
 }
 
+// Whether rows are cut into chunks, given a workspace: not short ones, which the row kernel
+// reads twice in the time of the finish kernel, whose workgroup per sequence folds eight
+// positions at a time and alone re-reads the chunks with possible ties. us, cut / whole, at
+// N(0, 2) logits (N(0, 0.2): ties possible): vocab 8000, 1 x 8 positions 7.2 / 9.3 (7.6 /
+// 9.1), 4 x 64 16.4 / 9.8 (34 / 9.5); 24576, 16 x 8 8.7 / 14.1 (21.1 / 14.0), 4 x 64 19.2 /
+// 13.5 (31.5 / 13.7); 32001 (no multiple of 8, read element by element), 16 x 8 9.0 / 29.7
+// (14.4 / 29.6); 152064, 16 x 8 13.7 / 53.1.
+inline bool unmask_cut(int vocab, int positions) {
+  return vocab > (vocab % 8 != 0 ? 1 : positions > 32 ? 6 : 3) * kChunk;
+}
+
 // Chunks of a row, one more where a row start off a 16-byte boundary can need it.
 inline int64_t unmask_chunks(int vocab) { return (static_cast<int64_t>(vocab) + 7 + kChunk - 1) / kChunk; }
 
@@ -443,7 +454,9 @@ extern "C" int fdllm_unmask_workspace_size(int vocab, int batch, int num_positio
   using namespace fdllm;
   FDLLM_CHECK_ARG(bytes != nullptr && vocab > 0 && batch >= 0 && num_positions >= 0 && num_positions <= 64,
                   "fdllm_unmask_workspace_size: need 0 <= num_positions <= 64 and vocab > 0");
-  *bytes = static_cast<size_t>(unmask_chunks(vocab)) * batch * num_positions * sizeof(float4);
+  *bytes = 0;
+  if (unmask_cut(vocab, num_positions))
+    *bytes = static_cast<size_t>(unmask_chunks(vocab)) * batch * num_positions * sizeof(float4);
   return FDLLM_OK;
 }
 
@@ -484,7 +497,7 @@ int unmask_launch(const char* what, const void* logits, int64_t logits_stride_b,
   hipStream_t s = static_cast<hipStream_t>(stream);
   a.parts = nullptr;
   a.n_chunks = 0;
-  if (chunked) {
+  if (chunked && unmask_cut(vocab, num_positions)) {
     const int64_t chunks = unmask_chunks(vocab);
     const size_t need = static_cast<size_t>(chunks) * batch * num_positions * sizeof(float4);
     if (workspace == nullptr || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) {

@@ -475,8 +475,8 @@ int fdllm_unmask_step(const void* logits, int64_t logits_stride_b, int64_t logit
                       int64_t* row_tok, float* row_conf, int32_t* counts,
                       int batch, int num_positions, int dtype, void* stream);
 
-/* fdllm_unmask_step with device scratch: each logits row is cut over several
- * workgroups and read once. The same outputs (row_conf may differ where a sum in another
+/* fdllm_unmask_step with device scratch: each long logits row is cut over several
+ * workgroups and read once (the workspace size is 0 where rows are short). The same outputs (row_conf may differ where a sum in another
  * order crosses a rounding boundary of the logits' type). `workspace`
  * (fdllm_unmask_workspace_size bytes, 16-byte aligned) needs no initialisation; calls that
  * may overlap in time, or whose two kernels may alternate on one stream (launched by

@@ -155,7 +155,7 @@ def _step_without_workspace(raw, x, mask_id, threshold):
 
 
 @pytest.mark.parametrize("workspace", [True, False])
-@pytest.mark.parametrize("V", [1000, 9001])
+@pytest.mark.parametrize("V", [1000, 9001, 24584])
 def test_rows_without_a_finite_probability(gpu, V, workspace):
     """Rows of -inf, of NaN and with one NaN or +inf among finite logits: the token lies in
     the vocabulary (0 where nothing is above -inf, as argmax over NaN), the position stays
@@ -183,12 +183,13 @@ def test_rows_without_a_finite_probability(gpu, V, workspace):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_sums_of_exponentials_carry_no_bias(gpu, dtype):
-    """A chunk's sum of exp(l - max), which the kernel leaves in the workspace, against 64
-    bits. Each of the 8192 terms has a relative error under 2^-22 and the fp32 additions one
-    of 2^-24 at most, 13 deep; their signs vary, so a row is off by some 1e-7 at most, and
-    the mean over 512 rows by 1e-8. A systematic error of the terms (log2 e rounded to 24
-    bits: 1.3e-8 of |l - max|, about 8 here) shows in that mean, at 4e-8 and more."""
-    B, L, V = 64, 8, 8000  # one chunk per row, starts on 16-byte boundaries
+    """The chunks' sums of exp(l - max), which the kernel leaves in the workspace, against 64
+    bits. Each of a chunk's 8192 terms has a relative error under 2^-22 and the fp32
+    additions one of 2^-24 at most, 13 deep; their signs vary, so a chunk is off by some 1e-7
+    at most, and the mean over 512 rows by 1e-8. A systematic error of the terms (log2 e
+    rounded to 24 bits: 1.3e-8 of |l - max|, about 8 here) shows in that mean, at 4e-8 and
+    more."""
+    B, L, V = 64, 8, 40960  # five whole chunks per row, and one for rows off a 16-byte boundary
     raw = (torch.randn(B, L, V, generator=torch.Generator().manual_seed(4)) * 2).to(dtype).to(gpu)
     x = torch.full((B, L), V, dtype=torch.int64, device=gpu)
     sc, need = ops.UnmaskScratch(B, L, gpu), ctypes.c_size_t(0)
@@ -198,8 +199,8 @@ def test_sums_of_exponentials_carry_no_bias(gpu, dtype):
         raw.data_ptr(), raw.stride(0), raw.stride(1), V, 0, 0, x.data_ptr(), x.stride(0), None, V, 2.0, -1,
         sc.row_tok.data_ptr(), sc.row_conf.data_ptr(), sc.counts.data_ptr(), B, L, _ffi.dtype_code(dtype),
         ws.data_ptr(), need.value, _ffi.stream_ptr(gpu)), "fdllm_unmask_step_ws")
-    got = ws.view(B, L, 4)  # (max, sum, index, near) per chunk
-    r = raw.double()
+    got = ws.view(B, L, -1, 4)[:, :, :5]  # (max, sum, index, near) per chunk
+    r = raw.view(B, L, 5, 8192).double()
     top = r.amax(dim=-1)
     assert torch.equal(got[..., 0].double(), top)
     err = got[..., 1].double() / torch.exp(r - top[..., None]).sum(dim=-1) - 1
@@ -207,7 +208,7 @@ def test_sums_of_exponentials_carry_no_bias(gpu, dtype):
     assert abs(float(err.mean())) < 2e-8 and float(err.abs().max()) < 5e-7
 
 
-@pytest.mark.parametrize("V", [1, 1000, 4099, 32001])
+@pytest.mark.parametrize("V", [1, 1000, 8192, 8193, 24576, 24584, 32001])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_step_without_a_workspace(gpu, V, dtype):
     """The two forms of the step choose the same tokens; confidences within one ulp of the
