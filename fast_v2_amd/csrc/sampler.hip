@@ -13,7 +13,7 @@
 // unmask_finish_kernel, one workgroup per sequence, folds the chunks of each position,
 // re-reads only the chunks in which a tie is possible, and applies the unmask rule.
 // What bounds it: the one read of the logits. 16 x 8 positions of 152064 bf16 logits
-// (38.9 MB): 9.8 us (4.0 TB/s) + 4.9 us for the finish, against 50.0 us (128 workgroups, an
+// (38.9 MB): 10.4 us (3.7 TB/s) + 4.4 us for the finish, against 50.0 us (128 workgroups, an
 // online rescale chain per thread and the second read) + 4.4 us for the form below.
 // 8192 logits per workgroup (four 16-byte loads per thread in flight, 2432 workgroups)
 // keep every compute unit at eight workgroups.

@@ -15,7 +15,10 @@
 //     compute units, 152064 are 951. Smaller ones take BN = 64 and are cut over K until the
 //     compute units have a workgroup each; the parts meet as fp32 partials (device-coherent
 //     stores, one arrival counter per tile), which the last workgroup to arrive adds in
-//     range order, so the result does not depend on which that was.
+//     range order, so the result does not depend on which that was. Layers of 129 to 256
+//     tiles are one round that leaves up to half of the compute units idle (a K range of a
+//     tile each would be two rounds); utils/linear_layers.py leaves those to the library
+//     where that is faster.
 // The tile is handed to the epilogue as 8-column blocks of its two halves (columns c and
 // c + BN / 2 of one row), which makes a gate / up pair or a RoPE pair one work item.
 //
